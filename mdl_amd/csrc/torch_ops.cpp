@@ -1562,12 +1562,17 @@ Tensor clip_sparse_grad_norm_(TensorList replicated, TensorList sharded, double 
   Tensor sumsq = at::empty({2}, f32), norm = at::empty({1}, f32), coef = at::empty({1}, f32);
   const size_t wsb = mdl_sumsq_workspace_bytes((int32_t)std::max(rs.size(), ss.size()));
   Tensor ws = workspace(wsb, dev);
-  check(mdl_sumsq(rs.empty() ? nullptr : sd, (int32_t)rs.size(), sumsq.data_ptr<float>(), ws.data_ptr(), wsb, s),
-        "mdl_sumsq");
-  check(mdl_sumsq(ss.empty() ? nullptr : sd + rs.size(), (int32_t)ss.size(), sumsq.data_ptr<float>() + 1,
-                  ws.data_ptr(), wsb, s),
-        "mdl_sumsq");
-  check(mdl_clip_coef(sumsq.data_ptr<float>(), 2, (float)max_norm, norm.data_ptr<float>(), coef.data_ptr<float>(), s),
+  // a list without gradients adds nothing to the norm and launches nothing
+  // (both empty: one sum of no spans)
+  int32_t lists = 0;
+  auto sum_list = [&](const std::vector<mdl_span>& spans, const mdl_span* at) {
+    check(mdl_sumsq(spans.empty() ? nullptr : at, (int32_t)spans.size(), sumsq.data_ptr<float>() + lists++,
+                    ws.data_ptr(), wsb, s),
+          "mdl_sumsq");
+  };
+  if (!rs.empty()) sum_list(rs, sd);
+  if (!ss.empty() || rs.empty()) sum_list(ss, sd + rs.size());
+  check(mdl_clip_coef(sumsq.data_ptr<float>(), lists, (float)max_norm, norm.data_ptr<float>(), coef.data_ptr<float>(), s),
         "mdl_clip_coef");
   if (!all.empty()) check(mdl_scale(sd, (int32_t)all.size(), coef.data_ptr<float>(), s), "mdl_scale");
   return norm.reshape({});
