@@ -428,6 +428,27 @@ int mdl_backward_apply(const mdl_feature* feats, int32_t num_features,
                        uint32_t classes, void* stream);
 
 /*
+ * mdl_backward_sort / mdl_backward_count with hints about the order the
+ * entries come in; a hint decides how the call sorts, never what it gives.
+ * MDL_SORT_BY_TABLE: the live entries come table by table, each table's in
+ * one stretch (a grouped lookup whose tables are read by one feature each),
+ * short enough that sorting tiles and merging those that overlap beats the
+ * radix passes.  mdl_sort_hints says so from each table's entry count (a
+ * host array; the counts of a typical batch do).
+ */
+#define MDL_SORT_BY_TABLE 1u
+uint32_t mdl_sort_hints(const int64_t* table_entries, int32_t num_tables);
+int mdl_backward_sort_hinted(const mdl_table* tables, int32_t num_tables, int32_t max_dim,
+                             uint32_t* sort_keys, uint32_t* sort_payload, int64_t n,
+                             const int64_t* count, int32_t key_bits, uint32_t hints,
+                             void* workspace, size_t workspace_bytes, void* stream);
+int mdl_backward_count_hinted(const mdl_table* tables, int32_t num_tables, int32_t max_dim,
+                              uint32_t* sort_keys, uint32_t* sort_payload, int64_t n,
+                              const int64_t* count, int32_t key_bits, uint32_t hints,
+                              int64_t* unique_range, void* workspace, size_t workspace_bytes,
+                              void* stream);
+
+/*
  * Squared 2-norm of the coalesced gradient of every table,
  *   *sumsq = sum over distinct (table, row) of sum_j g[row, j]^2,
  * after mdl_backward_sort and with the same arguments and workspace (the

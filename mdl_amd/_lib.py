@@ -139,6 +139,8 @@ SIGNATURES: dict[str, tuple] = {
         [_P, _I32, _P, _I32, _I32, _P, _P, _I64, _P, _I32, _P, _F, _F, _P, _P, _SZ, _U32, _P],
     ),
     "mdl_backward_sort": (_I32, [_P, _I32, _I32, _P, _P, _I64, _P, _I32, _P, _SZ, _P]),
+    "mdl_sort_hints": (_U32, [_P, _I32]),
+    "mdl_backward_sort_hinted": (_I32, [_P, _I32, _I32, _P, _P, _I64, _P, _I32, _U32, _P, _SZ, _P]),
     "mdl_backward_apply": (
         _I32,
         [_P, _I32, _P, _I32, _I32, _P, _P, _I64, _I32, _P, _F, _F, _P, _P, _SZ, _U32, _P],
@@ -152,6 +154,7 @@ SIGNATURES: dict[str, tuple] = {
     "mdl_clip_coef": (_I32, [_P, _I32, _F, _P, _P, _P]),
     "mdl_scale": (_I32, [_P, _I32, _P, _P]),
     "mdl_backward_count": (_I32, [_P, _I32, _I32, _P, _P, _I64, _P, _I32, _P, _P, _SZ, _P]),
+    "mdl_backward_count_hinted": (_I32, [_P, _I32, _I32, _P, _P, _I64, _P, _I32, _U32, _P, _P, _SZ, _P]),
     "mdl_backward_coalesce": (
         _I32,
         [_P, _I32, _P, _I32, _I32, _P, _P, _I64, _I32, _P, _P, _P, _P, _P, _SZ, _U32, _P],

@@ -24,6 +24,7 @@
 #include <mutex>
 
 #include "common.cuh"
+#include "tile_sort.cuh"
 
 namespace mdl {
 
@@ -69,17 +70,32 @@ struct BwdWs {
   float* chunk_ss;        // [max_chunks] squared norms of the runs finished per chunk
 };
 
-// Entries one slot walks in a full chunk: kSlotRun for a big call; a small
-// one takes shorter slices (down to 16) so that its chunks -- one wave each
-// -- still give every SIMD a few (about 4096 chunks of 8 slots).
+// Entries one slot walks in a full chunk: kSlotRun for a big call; a smaller
+// one takes shorter slices (down to kSlotRunMin) so that its chunks -- one
+// wave each -- still give every SIMD a few.
+constexpr int kSlotRunMin = 16;
+constexpr int64_t kSlotTarget = 32768;
 static inline int slot_run_for(int64_t n) {
+  const int64_t r = n / kSlotTarget;
+  return (int)(r < kSlotRunMin ? kSlotRunMin : (r > kSlotRun ? kSlotRun : r));
+}
+
+// Entries of a full chunk at least, whatever its table's slots: what bounds
+// the chunk count, and with it the workspace.
+static inline int chunk_min_for(int64_t n) {
   const int64_t r = n / 32768;
   return (int)(r < 16 ? 16 : (r > kSlotRun ? kSlotRun : r));
 }
 
-// A chunk holds at least slot_run entries unless it is its table's last, so
-// a call of n entries has at most ceil(n / slot_run) + T chunks.  That count
-// wobbles between 32 K and 34 K chunks while slot_run grows with n; the bound
+// Chunk sizes of a call, as the plan kernels take them.
+struct ChunkRule {
+  int slot_run, chunk_min;
+};
+static inline ChunkRule chunk_rule(int64_t n) { return {slot_run_for(n), chunk_min_for(n)}; }
+
+// A chunk holds at least chunk_min entries unless it is its table's last, so
+// a call of n entries has at most ceil(n / chunk_min) + T chunks.  That count
+// wobbles between 32 K and 34 K chunks while chunk_min grows with n; the bound
 // below covers it and never decreases with n, so a workspace sized for the
 // largest call serves every smaller one.
 static inline int64_t max_chunks_for(int64_t n, int32_t T) {
@@ -134,11 +150,11 @@ __device__ __forceinline__ int table_variant(const mdl_table& tb) {
 }
 
 // Entries per chunk of a table: slot_run per slot, one slot per L lanes.
-__device__ __forceinline__ int64_t table_chunk_len(const mdl_table& tb, int slot_run) {
+__device__ __forceinline__ int64_t table_chunk_len(const mdl_table& tb, ChunkRule rule) {
   const int c = variant_elems(table_variant(tb));
   const int64_t g = kWave / lanes_for(tb.dim > 0 ? tb.dim : 1, c);
-  const int64_t cb = (int64_t)slot_run * g;
-  return cb < kChunkMax ? cb : kChunkMax;
+  const int64_t cb = (int64_t)rule.slot_run * g;
+  return cb < rule.chunk_min ? rule.chunk_min : (cb < kChunkMax ? cb : kChunkMax);
 }
 
 // Bounds of every table in the sorted keys: block 2t finds the first key >=
@@ -192,13 +208,13 @@ __global__ __launch_bounds__(256) void bwd_desc_kernel(const mdl_table* __restri
                                                        int64_t* __restrict__ chunk_base,
                                                        int64_t* __restrict__ total,
                                                        ChunkDesc* __restrict__ desc, int64_t max_chunks,
-                                                       int slot_run) {
+                                                       ChunkRule rule) {
   __shared__ int64_t s_part[256 / kWave];
   const int32_t t = blockIdx.x;
   const int lane = lane_id(), w = threadIdx.x / kWave;
   int64_t before = 0;
   for (int32_t q = threadIdx.x; q < t; q += blockDim.x) {
-    const int64_t cq = table_chunk_len(tables[q], slot_run);
+    const int64_t cq = table_chunk_len(tables[q], rule);
     const int64_t sq = table_start[q], eq = table_end[q];
     before += ((eq > sq ? eq : sq) - sq + cq - 1) / cq;
   }
@@ -213,7 +229,7 @@ __global__ __launch_bounds__(256) void bwd_desc_kernel(const mdl_table* __restri
   for (int q = 0; q < 256 / kWave; ++q) base += s_part[q];
   const int64_t lo = table_start[t], hi_raw = table_end[t];
   const int64_t hi = hi_raw > lo ? hi_raw : lo;
-  const int64_t cb = table_chunk_len(tables[t], slot_run);
+  const int64_t cb = table_chunk_len(tables[t], rule);
   const int64_t room = max_chunks - base;
   const int64_t nch_all = (hi - lo + cb - 1) / cb;
   const int64_t nch = nch_all < room ? nch_all : (room > 0 ? room : 0);
@@ -229,6 +245,79 @@ __global__ __launch_bounds__(256) void bwd_desc_kernel(const mdl_table* __restri
     d.begin = b;
     desc[base + j] = d;
   }
+}
+
+// Sort and chunk plan of a call of one tile in one launch: the block sorts
+// the entries, finds every table's bounds in LDS and writes the descriptors
+// that bwd_bounds_kernel and bwd_desc_kernel write for larger calls.
+__global__ __launch_bounds__(kTileThreads) void tile_plan_kernel(TileSortArgs a, int64_t* __restrict__ table_start,
+                                                                 int64_t* __restrict__ table_end,
+                                                                 int64_t* __restrict__ chunk_base,
+                                                                 int64_t* __restrict__ total,
+                                                                 ChunkDesc* __restrict__ desc, int64_t max_chunks,
+                                                                 ChunkRule rule) {
+  __shared__ TileStage st;
+  __shared__ int32_t s_lo[kTileThreads], s_hi[kTileThreads], s_base[kTileThreads];
+  __shared__ int32_t s_wave[kTileWaves];
+  const int64_t n = entries_present(a.n_cap, a.n_dev);
+  uint32_t live = 0u, key_min = 0u;
+  if (n > 0) sort_tile(a, 0, n, st, &live, &key_min);
+  const int tid = threadIdx.x, w = tid / kWave, lane = lane_id();
+  // entries below a key
+  auto below = [&](uint64_t key) {
+    if (key <= key_min) return 0;
+    const uint64_t off = key - key_min;
+    return off > 0xffffffffull ? (int)live : count_before(st.key, 0, (int)live, (uint32_t)off, false);
+  };
+  int carry = 0;
+  for (int32_t t0 = 0; t0 < a.T; t0 += kTileThreads) {
+    const int32_t t = t0 + tid;
+    int lo = 0, hi = 0, nch = 0;
+    if (t < a.T) {
+      const mdl_table& tb = a.tables[t];
+      lo = below((uint64_t)tb.row_base);
+      hi = below((uint64_t)tb.row_base + (uint64_t)tb.num_rows);
+      table_start[t] = lo;
+      table_end[t] = hi;
+      const int cb = (int)table_chunk_len(tb, rule);
+      nch = ((hi > lo ? hi : lo) - lo + cb - 1) / cb;
+    }
+    int x = nch;  // inclusive scan of the chunk counts
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const int o = shfl_i(x, lane >= d ? lane - d : lane);
+      if (lane >= d) x += o;
+    }
+    if (lane == kWave - 1) s_wave[w] = x;
+    __syncthreads();
+    int before = carry, all = 0;
+#pragma unroll
+    for (int q = 0; q < kTileWaves; ++q) {
+      before += q < w ? s_wave[q] : 0;
+      all += s_wave[q];
+    }
+    s_lo[tid] = lo;
+    s_hi[tid] = hi > lo ? hi : lo;
+    s_base[tid] = before + x - nch;
+    __syncthreads();
+    const int in_round = a.T - t0 < kTileThreads ? a.T - t0 : kTileThreads;
+    for (int j = w; j < in_round; j += kTileWaves) {
+      const int cb = (int)table_chunk_len(a.tables[t0 + j], rule);
+      const int b0 = s_lo[j], b1 = s_hi[j];
+      const int64_t base = s_base[j];
+      if (lane == 0) chunk_base[t0 + j] = base < max_chunks ? base : max_chunks;
+      for (int c = lane; b0 + c * cb < b1 && base + c < max_chunks; c += kWave) {
+        ChunkDesc d;
+        d.table = t0 + j;
+        d.len = b1 - (b0 + c * cb) < cb ? b1 - (b0 + c * cb) : cb;
+        d.begin = b0 + c * cb;
+        desc[base + c] = d;
+      }
+    }
+    carry += all;
+    __syncthreads();  // the next round restages the LDS
+  }
+  if (tid == 0) *total = carry < max_chunks ? carry : max_chunks;
 }
 
 // Heads (first entry of a run) per chunk, for the coalesced layout.
@@ -256,10 +345,10 @@ __global__ __launch_bounds__(256) void count_heads_kernel(const int64_t* __restr
 __global__ void unique_range_end_kernel(int32_t T, const int64_t* table_start, const int64_t* table_end,
                                         const int64_t* chunk_base, const int64_t* head_base,
                                         const mdl_table* __restrict__ tables, int64_t* unique_range,
-                                        int slot_run) {
+                                        ChunkRule rule) {
   for (int32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < T; t += gridDim.x * blockDim.x) {
     const int64_t lo = table_start[t], hi = table_end[t];
-    const int64_t cb = table_chunk_len(tables[t], slot_run);
+    const int64_t cb = table_chunk_len(tables[t], rule);
     const int64_t nch = (hi - lo + cb - 1) / cb;
     unique_range[2 * t] = head_base[chunk_base[t]];
     unique_range[2 * t + 1] = head_base[chunk_base[t] + nch];
@@ -986,16 +1075,77 @@ static int plan(const mdl_table* tables, int32_t T, const uint32_t* sk, int64_t 
                      w.table_start, w.table_end);
   MDL_CHECK_LAUNCH("bwd_bounds_kernel");
   hipLaunchKernelGGL(bwd_desc_kernel, dim3((unsigned)T), dim3(256), 0, s, tables, T, w.table_start, w.table_end,
-                     w.chunk_base, w.num_chunks, w.desc, max_chunks_for(n, T), slot_run_for(n));
+                     w.chunk_base, w.num_chunks, w.desc, max_chunks_for(n, T), chunk_rule(n));
   MDL_CHECK_LAUNCH("bwd_desc_kernel");
   return MDL_OK;
 }
 
+// How a call of n entries is sorted.  The radix sort takes three launches per
+// 8-bit pass; up to its work those launches are what it costs, so short calls
+// sort their tiles in LDS and merge them by rank (tile_sort.cuh), and a call
+// of one tile takes its chunk plan along.
+// Sort + plan, radix -> tiles (4096 entries each):
+//   3 K entries of 10 tables 37 -> 18 us; 32 K of one table (8 tiles, every
+//   pair overlapping) 38 -> 30; 393 K of 32 tables 59 -> 31; 131 K of 8 tables
+//   50 -> 32; 893 K of 64 tables, 24 of 34 K, 58 -> 51; 3.3 M of 200 tables of
+//   16 K 117 -> 98.
+// A merge costs about 1 us per two overlapping tiles, so entries in an order
+// the call does not know merge up to kMergeFreeTiles tiles; a call hinted to
+// come table by table has every table short enough (mdl_sort_hints): at
+// kHintLongest tiles a table, or kHintPairs overlapping pairs in all, the two
+// sorts take about the same time.
+constexpr int64_t kMergeFreeTiles = 12;
+constexpr int64_t kHintLongest = 10, kHintPairs = 16384;
+static bool sorts_by_tiles(int64_t n, int32_t key_bits, uint32_t hints) {
+  if (key_bits <= 0 || key_bits > 32) return false;
+  const int64_t tiles = merge_tiles(n);
+  return tiles <= kMergeFreeTiles || ((hints & MDL_SORT_BY_TABLE) && tiles <= kMaxMergeTiles);
+}
+
 static int prepare(const mdl_table* tables, int32_t T, int32_t max_dim, uint32_t* keys, uint32_t* payload,
-                   int64_t n, const int64_t* n_dev, int32_t key_bits, void* ws, size_t ws_bytes, hipStream_t s,
-                   BwdWs* w, const uint32_t** sk, const uint32_t** sv) {
+                   int64_t n, const int64_t* n_dev, int32_t key_bits, uint32_t hints, void* ws, size_t ws_bytes,
+                   hipStream_t s, BwdWs* w, const uint32_t** sk, const uint32_t** sv) {
   const size_t need = carve(w, ws, n, T, max_dim);
   if (ws_bytes < need) return fail(MDL_ERR_WORKSPACE, "backward: workspace too small");
+  if (sorts_by_tiles(n, key_bits, hints)) {
+    // The sorted pairs end where the radix passes would leave them (the
+    // calls that follow the sort derive that from key_bits).
+    const bool in_alt = sort_pass_count(key_bits) & 1;
+    const int64_t tiles = merge_tiles(n);
+    TileSortArgs a;
+    a.tables = tables;
+    a.T = T;
+    a.keys_in = keys;
+    a.vals_in = payload;
+    a.n_cap = n;
+    a.n_dev = n_dev;
+    a.tile_min = static_cast<uint32_t*>(w->sort_ws);
+    a.tile_max = a.tile_min + tiles;
+    a.tile_live = a.tile_max + tiles;
+    *sk = in_alt ? w->keys_alt : keys;
+    *sv = in_alt ? w->vals_alt : payload;
+    if (tiles == 1) {
+      a.keys_out = const_cast<uint32_t*>(*sk);
+      a.vals_out = const_cast<uint32_t*>(*sv);
+      a.tile_min = nullptr;
+      hipLaunchKernelGGL(tile_plan_kernel, dim3(1), dim3(kTileThreads), 0, s, a, w->table_start, w->table_end,
+                         w->chunk_base, w->num_chunks, w->desc, max_chunks_for(n, T), chunk_rule(n));
+      MDL_CHECK_LAUNCH("tile_plan_kernel");
+      return MDL_OK;
+    }
+    // tiles sorted into the other buffers, merged into the final ones
+    a.keys_out = in_alt ? keys : w->keys_alt;
+    a.vals_out = in_alt ? payload : w->vals_alt;
+    hipLaunchKernelGGL(tile_sort_kernel, dim3((unsigned)tiles), dim3(kTileThreads), 0, s, a);
+    MDL_CHECK_LAUNCH("tile_sort_kernel");
+    a.keys_in = a.keys_out;
+    a.vals_in = a.vals_out;
+    a.keys_out = const_cast<uint32_t*>(*sk);
+    a.vals_out = const_cast<uint32_t*>(*sv);
+    hipLaunchKernelGGL(rank_merge_kernel, dim3((unsigned)(tiles * kMergeParts)), dim3(kMergeThreads), 0, s, a);
+    MDL_CHECK_LAUNCH("rank_merge_kernel");
+    return plan(tables, T, *sk, n, n_dev, *w, s);
+  }
   int in_alt = 0;
   int rc = sort_pairs(keys, payload, w->keys_alt, w->vals_alt, n, n_dev, key_bits, w->sort_ws, w->sort_bytes,
                       &in_alt, s);
@@ -1203,16 +1353,33 @@ size_t mdl_backward_workspace_bytes(int64_t n, int32_t num_tables, int32_t max_d
   return bytes + 256;
 }
 
-int mdl_backward_sort(const mdl_table* tables, int32_t num_tables, int32_t max_dim, uint32_t* sort_keys,
-                      uint32_t* sort_payload, int64_t n, const int64_t* count, int32_t key_bits, void* workspace,
-                      size_t workspace_bytes, void* stream) {
+uint32_t mdl_sort_hints(const int64_t* table_entries, int32_t num_tables) {
+  int64_t pairs = 0, longest = 0;
+  for (int32_t t = 0; t < num_tables; ++t) {
+    const int64_t tiles = merge_tiles(table_entries[t]) + 1;  // a stretch starts anywhere in a tile
+    longest = tiles > longest ? tiles : longest;
+    pairs += tiles * tiles;
+  }
+  return longest <= kHintLongest && pairs <= kHintPairs ? MDL_SORT_BY_TABLE : 0u;
+}
+
+int mdl_backward_sort_hinted(const mdl_table* tables, int32_t num_tables, int32_t max_dim, uint32_t* sort_keys,
+                             uint32_t* sort_payload, int64_t n, const int64_t* count, int32_t key_bits,
+                             uint32_t hints, void* workspace, size_t workspace_bytes, void* stream) {
   int rc = validate_tables("mdl_backward_sort", num_tables, max_dim, n);
   if (rc) return rc;
   if (n == 0) return MDL_OK;
   BwdWs w;
   const uint32_t *sk, *sv;
-  return prepare(tables, num_tables, max_dim, sort_keys, sort_payload, n, count, key_bits, workspace,
+  return prepare(tables, num_tables, max_dim, sort_keys, sort_payload, n, count, key_bits, hints, workspace,
                  workspace_bytes, as_stream(stream), &w, &sk, &sv);
+}
+
+int mdl_backward_sort(const mdl_table* tables, int32_t num_tables, int32_t max_dim, uint32_t* sort_keys,
+                      uint32_t* sort_payload, int64_t n, const int64_t* count, int32_t key_bits, void* workspace,
+                      size_t workspace_bytes, void* stream) {
+  return mdl_backward_sort_hinted(tables, num_tables, max_dim, sort_keys, sort_payload, n, count, key_bits, 0u,
+                                  workspace, workspace_bytes, stream);
 }
 
 // Arguments of the calls that follow mdl_backward_sort: the sorted pairs are
@@ -1286,9 +1453,10 @@ int mdl_backward_adagrad(const mdl_feature* feats, int32_t num_features, const m
                             key_bits, bag_count, lr, eps, grad_scale, workspace, workspace_bytes, classes, stream);
 }
 
-int mdl_backward_count(const mdl_table* tables, int32_t num_tables, int32_t max_dim, uint32_t* sort_keys,
-                       uint32_t* sort_payload, int64_t n, const int64_t* count, int32_t key_bits,
-                       int64_t* unique_range, void* workspace, size_t workspace_bytes, void* stream) {
+int mdl_backward_count_hinted(const mdl_table* tables, int32_t num_tables, int32_t max_dim, uint32_t* sort_keys,
+                              uint32_t* sort_payload, int64_t n, const int64_t* count, int32_t key_bits,
+                              uint32_t hints, int64_t* unique_range, void* workspace, size_t workspace_bytes,
+                              void* stream) {
   int rc = validate_tables("mdl_backward_count", num_tables, max_dim, n);
   if (rc) return rc;
   hipStream_t s = as_stream(stream);
@@ -1299,8 +1467,8 @@ int mdl_backward_count(const mdl_table* tables, int32_t num_tables, int32_t max_
     MDL_CHECK_LAUNCH("unique_range_zero");
     return MDL_OK;
   }
-  rc = prepare(tables, num_tables, max_dim, sort_keys, sort_payload, n, count, key_bits, workspace, workspace_bytes,
-               s, &w, &sk, &sv);
+  rc = prepare(tables, num_tables, max_dim, sort_keys, sort_payload, n, count, key_bits, hints, workspace,
+               workspace_bytes, s, &w, &sk, &sv);
   if (rc) return rc;
   const int64_t mc = max_chunks_for(n, num_tables);
   int64_t* heads = (int64_t*)((char*)workspace + carve(&w, workspace, n, num_tables, max_dim));
@@ -1311,9 +1479,16 @@ int mdl_backward_count(const mdl_table* tables, int32_t num_tables, int32_t max_
   if (rc) return rc;
   hipLaunchKernelGGL(unique_range_end_kernel, dim3((unsigned)((num_tables + 255) / 256)), dim3(256), 0, s,
                      num_tables, w.table_start, w.table_end, w.chunk_base, w.head_base, tables, unique_range,
-                     slot_run_for(n));
+                     chunk_rule(n));
   MDL_CHECK_LAUNCH("unique_range_end_kernel");
   return MDL_OK;
+}
+
+int mdl_backward_count(const mdl_table* tables, int32_t num_tables, int32_t max_dim, uint32_t* sort_keys,
+                       uint32_t* sort_payload, int64_t n, const int64_t* count, int32_t key_bits,
+                       int64_t* unique_range, void* workspace, size_t workspace_bytes, void* stream) {
+  return mdl_backward_count_hinted(tables, num_tables, max_dim, sort_keys, sort_payload, n, count, key_bits, 0u,
+                                   unique_range, workspace, workspace_bytes, stream);
 }
 
 int mdl_backward_coalesce(const mdl_feature* feats, int32_t num_features, const mdl_table* tables,

@@ -632,6 +632,18 @@ struct CoalesceResult {
   CoalescedLayout layout;
 };
 
+// The sort's hints for a group: its entries come table by table when every
+// table is read by one feature.
+uint32_t sort_hints(const KeyGroup& g, const std::vector<mdl_feature>& feats) {
+  std::vector<int64_t> entries;
+  entries.reserve(g.recs.size());
+  for (const mdl_table& r : g.recs) {
+    if (r.feature < 0) return 0;
+    entries.push_back(feats[g.lo + r.feature].num_ids);
+  }
+  return mdl_sort_hints(entries.data(), (int32_t)entries.size());
+}
+
 // Sort, count and coalesce every key group of a call.  The counting kernels
 // of all groups go first (each group keeps its own workspace, which its
 // coalescing reduce reads), so a caller that needs the row counts on the host
@@ -706,8 +718,8 @@ CoalesceResult coalesce_groups(const Layout& L, std::vector<mdl_feature>& feats,
     l.p = reinterpret_cast<uint32_t*>(payload.data_ptr()) + first;
     l.ws = workspace(mdl_backward_workspace_bytes(n, Tg, L.max_dim), dev);
     l.classes = g.classes;
-    check(mdl_backward_count(l.td, Tg, L.max_dim, l.k, l.p, n, nullptr, L.key_bits, ur, l.ws.data_ptr(),
-                             (size_t)l.ws.numel(), s),
+    check(mdl_backward_count_hinted(l.td, Tg, L.max_dim, l.k, l.p, n, nullptr, L.key_bits, sort_hints(g, feats), ur,
+                                    l.ws.data_ptr(), (size_t)l.ws.numel(), s),
           "mdl_backward_count");
     launches.push_back(std::move(l));
   }
@@ -1772,14 +1784,14 @@ void packed_forward_(const Tensor& features, int64_t feature_offset, int64_t num
 
 void backward_sort_(const Tensor& tables, int64_t num_tables, const Tensor& keys, const Tensor& payload,
                     int64_t num_entries, const std::optional<Tensor>& count, int64_t count_offset, int64_t max_dim,
-                    int64_t key_bits, const Tensor& ws) {
+                    int64_t key_bits, const Tensor& ws, int64_t hints) {
   const at::Device dev = keys.device();
   const c10::DeviceGuard guard(dev);
-  check(mdl_backward_sort(reinterpret_cast<const mdl_table*>(tables.data_ptr()), (int32_t)num_tables, (int32_t)max_dim,
+  check(mdl_backward_sort_hinted(reinterpret_cast<const mdl_table*>(tables.data_ptr()), (int32_t)num_tables, (int32_t)max_dim,
                           reinterpret_cast<uint32_t*>(keys.data_ptr()), reinterpret_cast<uint32_t*>(payload.data_ptr()),
                           num_entries,
                           count.has_value() && count->defined() ? at_offset<int64_t>(*count, count_offset) : nullptr,
-                          (int32_t)key_bits, ws.data_ptr(), (size_t)ws.numel(), stream_of(dev)),
+                          (int32_t)key_bits, (uint32_t)hints, ws.data_ptr(), (size_t)ws.numel(), stream_of(dev)),
         "mdl_backward_sort");
 }
 
@@ -1805,20 +1817,10 @@ void fused_backward_rowwise_adagrad_(TensorList weights, TensorList accumulators
                                      const Tensor& payload, int64_t num_entries, const std::optional<Tensor>& count,
                                      int64_t count_offset, const std::optional<Tensor>& bag_count,
                                      const std::optional<Tensor>& grad_scale, const Tensor& ws, int64_t max_dim,
-                                     int64_t key_bits, int64_t classes, double lr, double eps) {
-  (void)weights;
-  (void)accumulators;
-  const at::Device dev = keys.device();
-  const c10::DeviceGuard guard(dev);
-  check(mdl_backward_adagrad(reinterpret_cast<const mdl_feature*>(features.data_ptr()), (int32_t)num_features,
-                             reinterpret_cast<const mdl_table*>(tables.data_ptr()), (int32_t)num_tables, (int32_t)max_dim,
-                             reinterpret_cast<uint32_t*>(keys.data_ptr()), reinterpret_cast<uint32_t*>(payload.data_ptr()),
-                             num_entries,
-                             count.has_value() && count->defined() ? at_offset<int64_t>(*count, count_offset) : nullptr,
-                             (int32_t)key_bits, ptr_or_null<float>(bag_count), (float)lr, (float)eps,
-                             ptr_or_null<float>(grad_scale), ws.data_ptr(), (size_t)ws.numel(), (uint32_t)classes,
-                             stream_of(dev)),
-        "mdl_backward_adagrad");
+                                     int64_t key_bits, int64_t classes, double lr, double eps, int64_t hints) {
+  backward_sort_(tables, num_tables, keys, payload, num_entries, count, count_offset, max_dim, key_bits, ws, hints);
+  backward_apply_(weights, accumulators, features, num_features, tables, num_tables, keys, payload, num_entries,
+                  bag_count, grad_scale, ws, max_dim, key_bits, classes, lr, eps);
 }
 
 void backward_sumsq_(const Tensor& features, int64_t num_features, const Tensor& tables, int64_t num_tables,
@@ -1903,7 +1905,7 @@ TORCH_LIBRARY(mdl_hip, m) {
         "Tensor(e!)[] outputs, int classes) -> ()",
         &packed_forward_);
   m.def("backward_sort_(Tensor tables, int num_tables, Tensor(a!) keys, Tensor(b!) payload, int num_entries, "
-        "Tensor? count, int count_offset, int max_dim, int key_bits, Tensor(c!) workspace) -> ()",
+        "Tensor? count, int count_offset, int max_dim, int key_bits, Tensor(c!) workspace, int hints=0) -> ()",
         &backward_sort_);
   m.def("backward_apply_(Tensor(a!)[] weights, Tensor(b!)[] accumulators, Tensor features, int num_features, "
         "Tensor tables, int num_tables, Tensor keys, Tensor payload, int num_entries, Tensor? bag_count, "
@@ -1912,7 +1914,7 @@ TORCH_LIBRARY(mdl_hip, m) {
   m.def("fused_backward_rowwise_adagrad_(Tensor(a!)[] weights, Tensor(b!)[] accumulators, Tensor features, "
         "int num_features, Tensor tables, int num_tables, Tensor(c!) keys, Tensor(d!) payload, int num_entries, "
         "Tensor? count, int count_offset, Tensor? bag_count, Tensor? grad_scale, Tensor(e!) workspace, "
-        "int max_dim, int key_bits, int classes, float lr, float eps) -> ()",
+        "int max_dim, int key_bits, int classes, float lr, float eps, int hints=0) -> ()",
         &fused_backward_rowwise_adagrad_);
   m.def("backward_sumsq_(Tensor features, int num_features, Tensor tables, int num_tables, Tensor keys, "
         "Tensor payload, int num_entries, Tensor? bag_count, Tensor(a!) sumsq, int slot, Tensor(b!) workspace, "

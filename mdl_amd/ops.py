@@ -789,6 +789,18 @@ def table_classes(tables: np.ndarray) -> int:
     return int(lib().mdl_table_classes(tables.ctypes.data, len(tables)))
 
 
+def sort_hints(tables: np.ndarray, entries: Sequence[int]) -> int:
+    """Hints of a group's backward sort (``mdl_sort_hints``): its entries come
+    table by table when every table is read by one feature, ``entries[f]`` of
+    them for feature f in a typical batch."""
+
+    users = tables["feature"]
+    if len(tables) == 0 or bool((users < 0).any()):
+        return 0
+    counts = np.ascontiguousarray(np.asarray(entries, dtype=np.int64)[users])
+    return int(lib().mdl_sort_hints(counts.ctypes.data, len(counts)))
+
+
 def lane_elems(dim: int, esize: int, vec: bool) -> int:
     """Elements one lane moves per row in the kernels (their width rule):
     one 16-byte vector of the weight type, doubled up to 8 elements while

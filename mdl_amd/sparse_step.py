@@ -67,6 +67,7 @@ class _KeyGroup:
     tables: np.ndarray
     tables_dev: Tensor
     bwd_classes: int
+    hints: int
     keys: Tensor
     payload: Tensor
     ws: Tensor
@@ -204,6 +205,7 @@ class SparseStep:
                 gs.tables["feature"] = -1
             gs.fwd_classes = ops.feature_classes(np.ascontiguousarray(fwd[0][g.lo: g.hi]))
             gs.bwd_classes = ops.table_classes(gs.tables)
+            gs.hints = ops.sort_hints(gs.tables, list(id_counts)[g.lo: g.hi])
             gs.feats_fwd_dev = ops.upload(f_fwd, self.device)
             gs.chunks_dev = ops.upload(ch, self.device)
             gs.n_chunks = nc
@@ -346,7 +348,7 @@ class SparseStep:
         for g, gs in enumerate(self.groups):
             count, at = self._count(g) if self.k == 1 else (None, 0)
             torch.ops.mdl_hip.backward_sort_(gs.tables_dev, len(gs.tables), gs.keys, gs.payload, self._n(), count, at,
-                                             self.plan.max_dim, self.plan.key_bits, gs.ws)
+                                             self.plan.max_dim, self.plan.key_bits, gs.ws, gs.hints)
 
     def apply(self, lr: float, eps: float, grad_scale: Tensor | None = None) -> None:
         """Segment reduction of duplicate rows + fused row-wise Adagrad
@@ -388,7 +390,7 @@ class SparseStep:
                 torch.ops.mdl_hip.fused_backward_rowwise_adagrad_(
                     self._weights, self._states, gs.feats_bwd_dev, len(gs.feats_bwd), gs.tables_dev, len(gs.tables),
                     gs.keys, gs.payload, self._n(), count, at, self.bag_count, None, gs.ws, self.plan.max_dim,
-                    self.plan.key_bits, gs.bwd_classes, float(lr), float(eps),
+                    self.plan.key_bits, gs.bwd_classes, float(lr), float(eps), gs.hints,
                 )
         else:
             self.sort()
