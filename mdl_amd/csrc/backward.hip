@@ -71,10 +71,17 @@ struct BwdWs {
 };
 
 // Entries one slot walks in a full chunk: kSlotRun for a big call; a smaller
-// one takes shorter slices (down to kSlotRunMin) so that its chunks -- one
-// wave each -- still give every SIMD a few.
-constexpr int kSlotRunMin = 16;
-constexpr int64_t kSlotTarget = 32768;
+// one takes shorter slices (one entry per kSlotTarget, down to kSlotRunMin),
+// since a wave's walk is a chain of memory round trips and a small call has
+// waves to spare.  Reduce launches at one entry per 16 K / 32 K / 64 K / 128 K:
+// 393 K entries of 32 fp32 tables x 64 58.3 / 57.2 / 51.1 / 53.8 us (54.1
+// with slices of 16 at least); 893 K of 64 bf16 tables 80.9 / 55.3 / 40.5 /
+// 40.8 (its norm pass 49.3 / 29.5 / 21.6 / 23.9); 262 K of one bf16 table
+// 27.1 / 19.5 / 16.5 / 16.4 (27.4 with slices of 16 at least); 131 K uniform
+// ids 22.2 / 19.7 / 19.6 / 19.7 (29.2).  Shorter slices leave more runs
+// crossing slots and chunks.
+constexpr int kSlotRunMin = 4;
+constexpr int64_t kSlotTarget = 65536;
 static inline int slot_run_for(int64_t n) {
   const int64_t r = n / kSlotTarget;
   return (int)(r < kSlotRunMin ? kSlotRunMin : (r > kSlotRun ? kSlotRun : r));
