@@ -169,48 +169,101 @@ __global__ __launch_bounds__(kGatherThreads) void bag_gather_kernel(
 constexpr int kScanThreads = 256;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kScanThreads * kScanItems;
+// A scan of up to kScanOneBlock lengths is one block's, in one launch.
+constexpr int kScanOneThreads = 1024;
+constexpr int kScanOneBlock = kScanOneThreads * kScanItems;
 
-template <typename T>
-__device__ T block_exclusive_scan(T v, T* smem, T* total) {
-  // smem: kScanThreads entries.
-  const int tid = threadIdx.x;
-  smem[tid] = v;
-  __syncthreads();
-  for (int d = 1; d < kScanThreads; d <<= 1) {
-    T o = tid >= d ? smem[tid - d] : T(0);
-    __syncthreads();
-    smem[tid] += o;
-    __syncthreads();
-  }
-  T incl = smem[tid];
-  if (total) *total = smem[kScanThreads - 1];
-  __syncthreads();
-  return incl - v;
+__device__ __forceinline__ int64_t shfl_i64(int64_t v, int src) {
+  const uint32_t lo = (uint32_t)shfl_i((int)(uint32_t)v, src), hi = (uint32_t)shfl_i((int)(v >> 32), src);
+  return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
-__global__ void scan_tile_sums(const int64_t* __restrict__ in, int64_t n, int64_t* __restrict__ sums) {
-  __shared__ int64_t smem[kScanThreads];
+// Exclusive scan of one value per thread over a block of kThreads: shuffles
+// inside each wave, one barrier for the wave totals (256 threads through LDS
+// alone took 16 barriers and half the scan's time).  smem holds a word per
+// wave.
+template <int kThreads>
+__device__ __forceinline__ int64_t block_exclusive_scan(int64_t v, int64_t* smem, int64_t* total) {
+  constexpr int kWaves = kThreads / kWave;
+  const int lane = lane_id(), w = threadIdx.x / kWave;
+  int64_t x = v;
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    const int64_t o = shfl_i64(x, lane >= d ? lane - d : lane);
+    if (lane >= d) x += o;
+  }
+  if (lane == kWave - 1) smem[w] = x;
+  __syncthreads();
+  int64_t before = 0, all = 0;
+#pragma unroll
+  for (int q = 0; q < kWaves; ++q) {
+    before += q < w ? smem[q] : 0;
+    all += smem[q];
+  }
+  if (total) *total = all;
+  __syncthreads();
+  return before + x - v;
+}
+
+// offsets[i + 1] = prefix + sum(in[0 .. i]) over this block's tile of
+// blockDim.x * kScanItems lengths from base.
+template <int kThreads>
+__device__ __forceinline__ void scan_tile(const int64_t* __restrict__ in, int64_t n, int64_t base, int64_t prefix,
+                                          int64_t* smem, int64_t* __restrict__ offsets) {
+  const int64_t first = base + (int64_t)threadIdx.x * kScanItems;
+  int64_t v[kScanItems];
+  int64_t s = 0;
+#pragma unroll
+  for (int k = 0; k < kScanItems; ++k) v[k] = first + k < n ? in[first + k] : 0;
+#pragma unroll
+  for (int k = 0; k < kScanItems; ++k) s += v[k];
+  int64_t ex = block_exclusive_scan<kThreads>(s, smem, nullptr) + prefix;
+#pragma unroll
+  for (int k = 0; k < kScanItems; ++k) {
+    ex += v[k];
+    if (first + k < n) offsets[first + k + 1] = ex;
+  }
+}
+
+__global__ __launch_bounds__(kScanOneThreads) void scan_one_block(const int64_t* __restrict__ in, int64_t n,
+                                                                  int64_t* __restrict__ offsets) {
+  __shared__ int64_t smem[kScanOneThreads / kWave];
+  if (threadIdx.x == 0) offsets[0] = 0;
+  scan_tile<kScanOneThreads>(in, n, 0, 0, smem, offsets);
+}
+
+__global__ __launch_bounds__(kScanThreads) void scan_tile_sums(const int64_t* __restrict__ in, int64_t n,
+                                                               int64_t* __restrict__ sums) {
+  __shared__ int64_t smem[kScanThreads / kWave];
   const int64_t base = (int64_t)blockIdx.x * kScanTile;
+  int64_t v[kScanItems];
   int64_t s = 0;
 #pragma unroll
   for (int k = 0; k < kScanItems; ++k) {
-    int64_t i = base + (int64_t)k * kScanThreads + threadIdx.x;
-    if (i < n) s += in[i];
+    const int64_t i = base + (int64_t)k * kScanThreads + threadIdx.x;
+    v[k] = i < n ? in[i] : 0;
   }
-  int64_t total;
-  block_exclusive_scan<int64_t>(s, smem, &total);
-  if (threadIdx.x == 0) sums[blockIdx.x] = total;
+#pragma unroll
+  for (int k = 0; k < kScanItems; ++k) s += v[k];
+  for (int m = 1; m < kWave; m <<= 1) s += shfl_i64(s, lane_id() ^ m);
+  if (lane_id() == 0) smem[threadIdx.x / kWave] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int64_t t = 0;
+    for (int q = 0; q < kScanThreads / kWave; ++q) t += smem[q];
+    sums[blockIdx.x] = t;
+  }
 }
 
 // Exclusive scan of the per-tile sums in place, one block, any count.
-__global__ void scan_sums_single(int64_t* __restrict__ sums, int64_t m) {
-  __shared__ int64_t smem[kScanThreads];
+__global__ __launch_bounds__(kScanThreads) void scan_sums_single(int64_t* __restrict__ sums, int64_t m) {
+  __shared__ int64_t smem[kScanThreads / kWave];
   int64_t carry = 0;
   for (int64_t base = 0; base < m; base += kScanThreads) {
     int64_t i = base + threadIdx.x;
     int64_t v = i < m ? sums[i] : 0;
     int64_t total;
-    int64_t ex = block_exclusive_scan<int64_t>(v, smem, &total);
+    int64_t ex = block_exclusive_scan<kScanThreads>(v, smem, &total);
     if (i < m) sums[i] = carry + ex;
     carry += total;
   }
@@ -219,35 +272,20 @@ __global__ void scan_sums_single(int64_t* __restrict__ sums, int64_t m) {
 // offsets[i+1] = sum(in[0..i]); offsets[0] = 0.  The tile's prefix is
 // sums[b] after scan_sums_single, or, with prefix_self (few tiles), the sum
 // of the raw tile sums before it, added up here: one launch fewer.
-__global__ void scan_tiles_final(const int64_t* __restrict__ in, int64_t n,
-                                 const int64_t* __restrict__ sums, int64_t* __restrict__ offsets,
-                                 int prefix_self) {
-  __shared__ int64_t smem[kScanThreads];
+__global__ __launch_bounds__(kScanThreads) void scan_tiles_final(const int64_t* __restrict__ in, int64_t n,
+                                                                 const int64_t* __restrict__ sums,
+                                                                 int64_t* __restrict__ offsets, int prefix_self) {
+  __shared__ int64_t smem[kScanThreads / kWave];
   int64_t tile_prefix;
   if (prefix_self) {
     int64_t p = 0;
     for (int64_t j = threadIdx.x; j < (int64_t)blockIdx.x; j += kScanThreads) p += sums[j];
-    block_exclusive_scan<int64_t>(p, smem, &tile_prefix);
+    block_exclusive_scan<kScanThreads>(p, smem, &tile_prefix);
   } else {
     tile_prefix = sums[blockIdx.x];
   }
-  const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
-  int64_t v[kScanItems];
-  int64_t s = 0;
-#pragma unroll
-  for (int k = 0; k < kScanItems; ++k) {
-    int64_t i = base + k;
-    v[k] = i < n ? in[i] : 0;
-    s += v[k];
-  }
-  int64_t ex = block_exclusive_scan<int64_t>(s, smem, nullptr) + tile_prefix;
   if (blockIdx.x == 0 && threadIdx.x == 0) offsets[0] = 0;
-#pragma unroll
-  for (int k = 0; k < kScanItems; ++k) {
-    int64_t i = base + k;
-    ex += v[k];
-    if (i < n) offsets[i + 1] = ex;
-  }
+  scan_tile<kScanThreads>(in, n, (int64_t)blockIdx.x * kScanTile, tile_prefix, smem, offsets);
 }
 
 static __global__ void zero_offset_kernel(int64_t* p) { *p = 0; }
@@ -344,6 +382,11 @@ int mdl_lengths_to_offsets(const int64_t* lengths, int64_t n, int64_t* offsets, 
   }
   if (workspace_bytes < mdl_offsets_workspace_bytes(n))
     return fail(MDL_ERR_WORKSPACE, "mdl_lengths_to_offsets: workspace too small");
+  if (n <= kScanOneBlock) {
+    hipLaunchKernelGGL(scan_one_block, dim3(1), dim3(kScanOneThreads), 0, s, lengths, n, offsets);
+    MDL_CHECK_LAUNCH("scan_one_block");
+    return MDL_OK;
+  }
   int64_t tiles = (n + kScanTile - 1) / kScanTile;
   int64_t* sums = static_cast<int64_t*>(workspace);
   hipLaunchKernelGGL(scan_tile_sums, dim3((unsigned)tiles), dim3(kScanThreads), 0, s, lengths, n, sums);
