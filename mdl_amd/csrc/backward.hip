@@ -45,10 +45,21 @@ enum { kHeadOpen = 1, kTailOpen = 2, kSingle = 4 };
 enum { kModeAdagrad = 0, kModeCoalesce = 1, kModeSumsq = 2 };
 
 // One chunk: entries [begin, begin + len) of the sorted array, all of table.
-struct ChunkDesc {
+// It carries what a wave would otherwise look up in turn -- the table's kernel
+// variant, its only feature (-1: several) and whether the chunk starts or ends
+// the table's stretch -- so that the table's and feature's records and the
+// chunk's keys load together, one round trip after the descriptor.
+// (8 M entries of 200 tables: reduce 573 -> 566 us, the step 1104.6 -> 1096.1.)
+enum { kTableFirst = 1, kTableLast = 2 };
+struct alignas(16) ChunkDesc {
   int32_t table;
-  int32_t len;
-  int64_t begin;
+  int32_t len_flags;  // len | (flags << 16) | (variant << 18)
+  uint32_t begin;
+  int32_t feature;
+  __host__ __device__ int len() const { return len_flags & 0xffff; }
+  __host__ __device__ bool first() const { return (len_flags >> 16) & kTableFirst; }
+  __host__ __device__ bool last() const { return (len_flags >> 16) & kTableLast; }
+  __host__ __device__ int variant() const { return len_flags >> 18; }
 };
 
 struct BwdWs {
@@ -156,6 +167,20 @@ __device__ __forceinline__ int table_variant(const mdl_table& tb) {
   return variant_of(tb.wdtype, tb.gdtype, table_vec(tb), tb.dim);
 }
 
+// Chunk j of table t (record tb) whose entries are [lo, hi), cut every cb.
+__device__ __forceinline__ ChunkDesc make_desc(const mdl_table& tb, int32_t t, int64_t lo, int64_t hi, int64_t cb,
+                                               int64_t j) {
+  const int64_t b = lo + j * cb;
+  const bool last = hi - b <= cb;
+  ChunkDesc d;
+  d.table = t;
+  d.len_flags = (int32_t)(last ? hi - b : cb) | (((j == 0 ? kTableFirst : 0) | (last ? kTableLast : 0)) << 16) |
+                (table_variant(tb) << 18);
+  d.begin = (uint32_t)b;
+  d.feature = tb.feature;
+  return d;
+}
+
 // Entries per chunk of a table: slot_run per slot, one slot per L lanes.
 __device__ __forceinline__ int64_t table_chunk_len(const mdl_table& tb, ChunkRule rule) {
   const int c = variant_elems(table_variant(tb));
@@ -245,12 +270,7 @@ __global__ __launch_bounds__(256) void bwd_desc_kernel(const mdl_table* __restri
     if (t == T - 1) *total = base + nch < max_chunks ? base + nch : max_chunks;
   }
   for (int64_t j = threadIdx.x; j < nch; j += blockDim.x) {
-    const int64_t b = lo + j * cb;
-    ChunkDesc d;
-    d.table = t;
-    d.len = (int32_t)(hi - b < cb ? hi - b : cb);
-    d.begin = b;
-    desc[base + j] = d;
+    desc[base + j] = make_desc(tables[t], t, lo, hi, cb, j);
   }
 }
 
@@ -313,13 +333,8 @@ __global__ __launch_bounds__(kTileThreads) void tile_plan_kernel(TileSortArgs a,
       const int b0 = s_lo[j], b1 = s_hi[j];
       const int64_t base = s_base[j];
       if (lane == 0) chunk_base[t0 + j] = base < max_chunks ? base : max_chunks;
-      for (int c = lane; b0 + c * cb < b1 && base + c < max_chunks; c += kWave) {
-        ChunkDesc d;
-        d.table = t0 + j;
-        d.len = b1 - (b0 + c * cb) < cb ? b1 - (b0 + c * cb) : cb;
-        d.begin = b0 + c * cb;
-        desc[base + c] = d;
-      }
+      for (int c = lane; b0 + c * cb < b1 && base + c < max_chunks; c += kWave)
+        desc[base + c] = make_desc(a.tables[t0 + j], t0 + j, b0, b1, cb, c);
     }
     carry += all;
     __syncthreads();  // the next round restages the LDS
@@ -330,7 +345,6 @@ __global__ __launch_bounds__(kTileThreads) void tile_plan_kernel(TileSortArgs a,
 // Heads (first entry of a run) per chunk, for the coalesced layout.
 __global__ __launch_bounds__(256) void count_heads_kernel(const int64_t* __restrict__ num_chunks,
                                                           const ChunkDesc* __restrict__ desc,
-                                                          const int64_t* __restrict__ table_start,
                                                           const uint32_t* __restrict__ keys, int64_t max_chunks,
                                                           int64_t* __restrict__ heads) {
   const int w = threadIdx.x / kWave, lane = lane_id();
@@ -341,10 +355,11 @@ __global__ __launch_bounds__(256) void count_heads_kernel(const int64_t* __restr
     return;
   }
   const ChunkDesc d = desc[c];
-  const int64_t t_begin = table_start[d.table];
   int cnt = 0;
-  for (int64_t e = d.begin + lane; e < d.begin + d.len; e += kWave)
-    cnt += (e == t_begin || keys[e] != keys[e - 1]) ? 1 : 0;
+  for (int i = lane; i < d.len(); i += kWave) {
+    const int64_t e = (int64_t)d.begin + i;
+    cnt += (i == 0 && d.first()) || keys[e] != keys[e - 1] ? 1 : 0;
+  }
   for (int m = 1; m < kWave; m <<= 1) cnt += __shfl_xor(cnt, m);
   if (lane == 0) heads[c] = cnt;
 }
@@ -392,8 +407,6 @@ struct BwdArgs {
   const uint32_t* keys;
   const uint32_t* vals;
   const float* bag_count;
-  const int64_t* table_start;
-  const int64_t* table_end;
   const int64_t* chunk_base;
   const int64_t* num_chunks;
   const ChunkDesc* desc;
@@ -441,10 +454,9 @@ struct Reducer {
   bool g_mean, g_pool_none;
   float scale;
 
-  __device__ Reducer(const BwdArgs& args, int32_t table) : a(args), t(table) {
+  __device__ Reducer(const BwdArgs& args, int32_t table, int32_t feature) : a(args), t(table), single(feature) {
     const mdl_table& tb = a.tables[t];
     dim = __builtin_amdgcn_readfirstlane(tb.dim);
-    single = __builtin_amdgcn_readfirstlane(tb.feature);
     W = (TW*)uni64b((int64_t)tb.weight);
     state = (float*)uni64b((int64_t)tb.state);
     row_base = uni64b(tb.row_base);
@@ -563,7 +575,7 @@ __device__ __forceinline__ void reduce_chunk_body(const BwdArgs& a, int64_t c, c
   constexpr bool coalesce = kMode == kModeCoalesce;
   const uint32_t kNone = 0xffffffffu;
   const int lane = lane_id();
-  const int len = d.len;
+  const int len = d.len();
   const int G = R.G, L = R.L, slot = R.slot;
   const bool head_open = st.key[0] == st.key[1];
   const bool tail_open = st.key[len + 1] == st.key[len];
@@ -770,7 +782,7 @@ __device__ void reduce_chunk_wide(const BwdArgs& a, int64_t c, const ChunkDesc& 
   constexpr int kSpan = kWave * C;
   constexpr int kU = 4;  // entries whose gradient rows load together
   const int lane = lane_id();
-  const int len = d.len;
+  const int len = d.len();
   const int nblk = (R.dim + kSpan - 1) / kSpan;
   const bool head_open = st.key[0] == st.key[1];
   const bool tail_open = st.key[len + 1] == st.key[len];
@@ -853,20 +865,35 @@ __device__ void reduce_chunk_wide(const BwdArgs& a, int64_t c, const ChunkDesc& 
 
 template <int kMode, typename TW, typename TG, int C>
 __device__ __forceinline__ void reduce_chunk(const BwdArgs& a, int64_t c, const ChunkDesc& d, ChunkStage& st) {
-  Reducer<kMode, TW, TG, C> R(a, d.table);
   const int lane = lane_id();
   const uint32_t kNone = 0xffffffffu;
-  const int len = d.len;
-  const int64_t t_begin = uni64b(a.table_start[d.table]);
-  const int64_t t_end = uni64b(a.table_end[d.table]);
-  for (int i = lane; i < len; i += kWave) {
-    st.key[i + 1] = a.keys[d.begin + i];
-    st.pay[i] = a.vals[d.begin + i];
+  const int len = d.len();
+  // The chunk's keys and payloads are requested before the records of its
+  // table and feature are waited for.
+  constexpr int kLoads = kChunkMax / kWave;
+  uint32_t k[kLoads], p[kLoads], edge = kNone;
+  const uint32_t* keys = a.keys + d.begin;
+  const uint32_t* vals = a.vals + d.begin;
+#pragma unroll
+  for (int q = 0; q < kLoads; ++q) {
+    if (q * kWave < len) {
+      const int i = q * kWave + lane < len ? q * kWave + lane : len - 1;
+      k[q] = ld_policy(keys + i);
+      p[q] = ld_policy(vals + i);
+    }
   }
-  if (lane == 0) {
-    st.key[0] = d.begin > t_begin ? a.keys[d.begin - 1] : kNone;
-    st.key[len + 1] = d.begin + len < t_end ? a.keys[d.begin + len] : kNone;
+  // lane 0: the key before the chunk; lane 1: the one after it
+  if (lane < 2 && !(lane == 0 ? d.first() : d.last())) edge = ld_policy(lane == 0 ? keys - 1 : keys + len);
+  Reducer<kMode, TW, TG, C> R(a, d.table, d.feature);
+#pragma unroll
+  for (int q = 0; q < kLoads; ++q) {
+    const int i = q * kWave + lane;
+    if (i < len) {
+      st.key[i + 1] = k[q];
+      st.pay[i] = p[q];
+    }
   }
+  if (lane < 2) st.key[lane == 0 ? 0 : len + 1] = edge;
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   if (kMode == kModeCoalesce) {
@@ -948,7 +975,7 @@ __device__ void fixup_chunk_wide(const BwdArgs& a, int64_t c, const ChunkDesc& d
 
 template <int kMode, typename TW, typename TG, int C>
 __device__ __forceinline__ void fixup_chunk(const BwdArgs& a, int64_t c, const ChunkDesc& d, int32_t flags) {
-  Reducer<kMode, TW, TG, C> R(a, d.table);
+  Reducer<kMode, TW, TG, C> R(a, d.table, d.feature);
   // Walk back over chunks that lie wholly inside the run to the chunk holding
   // its first entry (never past the table's first chunk).
   // The wave reads 64 chunks' flags per step (a Zipf head row spans many
@@ -1046,11 +1073,12 @@ __global__ MDL_OCCUPANCY __launch_bounds__(kBwdWaves * kWave) void bwd_reduce_ke
     flags = __builtin_amdgcn_readfirstlane(a.chunk_flags[c]);
     if (!(flags & kHeadOpen) || (flags & kSingle)) return;
   }
-  ChunkDesc d;
-  d.table = __builtin_amdgcn_readfirstlane(a.desc[c].table);
-  d.len = __builtin_amdgcn_readfirstlane(a.desc[c].len);
-  d.begin = uni64b(a.desc[c].begin);
-  const int v = table_variant(a.tables[d.table]);
+  ChunkDesc d = a.desc[c];
+  d.table = __builtin_amdgcn_readfirstlane(d.table);
+  d.len_flags = __builtin_amdgcn_readfirstlane(d.len_flags);
+  d.begin = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.begin);
+  d.feature = __builtin_amdgcn_readfirstlane(d.feature);
+  const int v = d.variant();
   if (v / kWidths != ClassOf<TW, TG, kVec>::value) return;  // another class's launch owns it
   if (kFixup) {
     with_width<TW, kVec>(v % kWidths, [&]<int C>() { fixup_chunk<kMode, TW, TG, C>(a, c, d, flags); });
@@ -1172,8 +1200,6 @@ static void fill_args(BwdArgs* a, const mdl_feature* feats, int32_t F, const mdl
   a->keys = sk;
   a->vals = sv;
   a->bag_count = bag_count;
-  a->table_start = w.table_start;
-  a->table_end = w.table_end;
   a->chunk_base = w.chunk_base;
   a->num_chunks = w.num_chunks;
   a->desc = w.desc;
@@ -1480,7 +1506,7 @@ int mdl_backward_count_hinted(const mdl_table* tables, int32_t num_tables, int32
   const int64_t mc = max_chunks_for(n, num_tables);
   int64_t* heads = (int64_t*)((char*)workspace + carve(&w, workspace, n, num_tables, max_dim));
   hipLaunchKernelGGL(count_heads_kernel, dim3((unsigned)((mc + 3) / 4)), dim3(256), 0, s, w.num_chunks, w.desc,
-                     w.table_start, sk, mc, heads);
+                     sk, mc, heads);
   MDL_CHECK_LAUNCH("count_heads_kernel");
   rc = mdl_lengths_to_offsets(heads, mc, w.head_base, w.scan_ws, w.scan_bytes, stream);
   if (rc) return rc;
