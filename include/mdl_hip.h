@@ -329,6 +329,16 @@ int mdl_sequence_forward(const mdl_feature* feature_host, const int64_t* ids,
 /* ---------------------------------------------------------------- sort --- */
 
 /*
+ * Window entries of the rows of several sequence features, for the offsets
+ * that pack their sort keys: clamped[i] = min(max(length, 0), caps[f]) for
+ * every row of feature f, the features' rows one after the other.  lengths
+ * (device addresses of int64 arrays), rows and caps are host arrays of
+ * num_features entries.
+ */
+int mdl_clamp_lengths(const uint64_t* lengths, const int64_t* rows, const int64_t* caps, int32_t num_features,
+                      int64_t* clamped, void* stream);
+
+/*
  * Stable LSD radix sort of (key, payload) pairs on the low key_bits bits,
  * 8 bits per pass, ping-ponging between (keys, payload) and (keys_alt,
  * payload_alt).  *result_in_alt (host) is set to 1 when the sorted pairs end

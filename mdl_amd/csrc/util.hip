@@ -344,6 +344,29 @@ __global__ __launch_bounds__(kGatherThreads) void bag_gather_kernel(
   if (error_count != nullptr && bad) atomicAdd(error_count, bad);
 }
 
+// Window entries of every row of up to kLenFeatures sequence features: the
+// rows' lengths clamped to [0, cap], one feature after the other.
+constexpr int kLenFeatures = 16;
+struct LenArgs {
+  const int64_t* lengths[kLenFeatures];
+  int64_t cap[kLenFeatures];
+  int64_t end[kLenFeatures];  // rows of the features up to and with this one
+  int32_t features;
+};
+
+__global__ __launch_bounds__(256) void clamp_lengths_kernel(LenArgs a, int64_t* __restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  int64_t start = 0;
+  for (int f = 0; f < a.features; ++f) {
+    if (i < a.end[f]) {
+      const int64_t n = a.lengths[f][i - start];
+      out[i] = n < 0 ? 0 : (n > a.cap[f] ? a.cap[f] : n);
+      return;
+    }
+    start = a.end[f];
+  }
+}
+
 static __global__ void zero_offset_kernel(int64_t* p) { *p = 0; }
 
 // Tiles whose prefix the final kernel adds up itself.
@@ -387,6 +410,33 @@ int mdl_bucketize(const int64_t* raw, const uint8_t* valid, int64_t n, int64_t n
                      valid, n, num_buckets, mode, validate_nonzero, out, error_count,
                      mod_magic_for(mode, num_buckets));
   MDL_CHECK_LAUNCH("bucketize_kernel");
+  return MDL_OK;
+}
+
+int mdl_clamp_lengths(const uint64_t* lengths, const int64_t* rows, const int64_t* caps, int32_t num_features,
+                      int64_t* clamped, void* stream) {
+  if (num_features < 0) return fail(MDL_ERR_INVALID, "mdl_clamp_lengths: negative count");
+  if (num_features > 0 && (!lengths || !rows || !caps || !clamped))
+    return fail(MDL_ERR_INVALID, "mdl_clamp_lengths: null pointer");
+  for (int32_t f0 = 0; f0 < num_features; f0 += kLenFeatures) {
+    LenArgs a{};
+    int64_t n = 0;
+    a.features = num_features - f0 < kLenFeatures ? num_features - f0 : kLenFeatures;
+    for (int32_t f = 0; f < a.features; ++f) {
+      if (rows[f0 + f] < 0) return fail(MDL_ERR_INVALID, "mdl_clamp_lengths: negative rows");
+      n += rows[f0 + f];
+      a.lengths[f] = reinterpret_cast<const int64_t*>(lengths[f0 + f]);
+      a.cap[f] = caps[f0 + f];
+      a.end[f] = n;
+    }
+    const int64_t blocks = (n + 255) / 256;
+    if (blocks > 0xffffff) return fail(MDL_ERR_UNSUPPORTED, "mdl_clamp_lengths: too many rows");
+    if (n > 0) {
+      hipLaunchKernelGGL(clamp_lengths_kernel, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), a, clamped);
+      MDL_CHECK_LAUNCH("clamp_lengths_kernel");
+    }
+    clamped += n;
+  }
   return MDL_OK;
 }
 

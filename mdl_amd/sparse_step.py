@@ -502,6 +502,8 @@ class SequenceStep:
         # Sort entries a row can hold: its window entries, at most the
         # window's width (none for an empty input).
         self.caps = [int(o.size(1)) if int(i.size(1)) > 0 else 0 for i, o in zip(self.ids, self.outputs)]
+        self._batch = np.array(self.batch, dtype=np.int64)
+        self._caps = np.array(self.caps, dtype=np.int64)
         for m in range(1, self.k):
             if [tuple(o.shape) for o in self.all_outputs[m]] != [tuple(o.shape) for o in self.outputs]:
                 raise ValueError("every micro-batch's windows need the shapes of the first's")
@@ -604,9 +606,12 @@ class SequenceStep:
         s = self._stream()
         # Entries each row keeps (its positions that reach the window), then
         # one scan over each key group's rows places them.
-        for f, ln in enumerate(self.lengths):
-            b0, b1 = int(self.row_base[f]), int(self.row_base[f + 1])
-            torch.clamp(ln, 0, self.caps[f], out=self.key_len[b0:b1])
+        lengths = np.array([ln.data_ptr() for ln in self.lengths], dtype=np.uint64)
+        check(
+            lib().mdl_clamp_lengths(lengths.ctypes.data, self._batch.ctypes.data, self._caps.ctypes.data, len(lengths),
+                                    self.key_len.data_ptr(), s),
+            "mdl_clamp_lengths",
+        )
         for gs in self.groups:
             nrows = gs.r1 - gs.r0
             check(
