@@ -931,6 +931,37 @@ __device__ __forceinline__ int64_t seq_src(const SeqArgs& a, int64_t len, int64_
   return k < a.in_len ? k : a.in_len - 1;
 }
 
+// Sort keys/payloads of the window entries (b, rel), rel in [0, len_b), of a
+// sequence feature: entry rel sits at window position p = out_len - len_b +
+// rel and reads input position seq_src(rel), so an input element that the
+// window repeats gets one entry per position.  Each wave writes those of the
+// positions it gathers, whose ids it has just read (a launch of their own
+// took 7 us per feature of 1024 x 2048 positions); the row's padding
+// positions take its unused entries rel >= len_b, sentinels.  Dense: entry
+// rel of row b at b * out_len + rel.  Packed (key_offsets): the row's first
+// cap = key_offsets[b + 1] - key_offsets[b] entries (at most out_len) at
+// key_offsets[b] + rel, so the sort sees no padding; a row longer than its
+// cap loses the rest, a shorter one fills it with sentinels.
+__device__ __forceinline__ void seq_keys(const SeqArgs& a, int64_t b, int64_t p0, int np, int64_t len) {
+  const int64_t start = a.out_len - len;
+  int64_t base = b * a.out_len, cap = a.out_len;
+  if (a.key_offsets != nullptr) {
+    base = a.key_offsets[b];
+    cap = a.key_offsets[b + 1] - base;
+    cap = cap < 0 ? 0 : (cap > a.out_len ? a.out_len : cap);
+  }
+  for (int i = lane_id(); i < np; i += kWave) {
+    const int64_t p = p0 + i;
+    const bool in_window = p >= start;
+    const int64_t rel = in_window ? p - start : len + p;
+    if (rel >= cap) continue;
+    const int64_t id = in_window ? a.ids[b * a.in_len + seq_src(a, len, rel)] : 0;
+    const bool valid = in_window && (uint64_t)id < (uint64_t)a.f.num_rows && id != a.f.padding_idx;
+    st_policy<kOutPolicy>(a.keys + base + rel, valid ? (uint32_t)(a.f.row_base + id) : a.sentinel);
+    st_policy<kOutPolicy>(a.payload + base + rel, valid ? (uint32_t)(a.f.payload_base + b * a.out_len + p) : 0u);
+  }
+}
+
 // One wave per chunk of kSeqRows output positions [p0, p0 + np) of one row
 // b of [batch, out_len]: the chunk's first nz positions are padding (zeros),
 // the rest hold the ids of one contiguous (oldest_to_newest) or reversed
@@ -1035,6 +1066,7 @@ __device__ __forceinline__ void seq_chunk(const SeqArgs& a, int64_t b, int64_t p
   }
   if (a.mask)
     for (int i = lane; i < np; i += kWave) a.mask[b * a.out_len + p0 + i] = i >= nz ? 1 : 0;
+  if (a.keys) seq_keys(a, b, p0, np, len);
   for (int m = 1; m < kWave; m <<= 1) bad += __shfl_xor(bad, m);
   if (lane == 0 && bad && a.error_count) atomicAdd(a.error_count, bad);
 }
@@ -1050,41 +1082,6 @@ __global__ MDL_OCCUPANCY __launch_bounds__(kFwdWaves * kWave) void sequence_kern
   const int64_t p0 = (wid - b * per_row) * kSeqRows;
   const int np = a.out_len - p0 < kSeqRows ? (int)(a.out_len - p0) : kSeqRows;
   with_width<TW, kVec>(width, [&]<int C>() { seq_chunk<TW, TO, C>(a, b, p0, np); });
-}
-
-// Sort keys/payloads of the window entries (b, rel), rel in [0, len_b), of a
-// sequence feature: entry rel sits at window position p = out_len - len_b +
-// rel and reads input position seq_src(rel), so an input element that the
-// window repeats gets one entry per position.  One block per kSeqKeys entries
-// of one row, so the row's length is one load.  Dense: entry rel of row b at
-// b * out_len + rel.  Packed (key_offsets): the row's first cap =
-// key_offsets[b + 1] - key_offsets[b] entries (at most out_len) at
-// key_offsets[b] + rel, so the sort sees no padding; a row longer than its
-// cap loses the rest, a shorter one fills it with sentinels.
-constexpr int kSeqKeys = 1024;
-
-__global__ __launch_bounds__(256) void sequence_keys_kernel(SeqArgs a) {
-  const int64_t per_row = (a.out_len + kSeqKeys - 1) / kSeqKeys;
-  const int64_t b = (int64_t)blockIdx.x / per_row;
-  const int64_t kb = ((int64_t)blockIdx.x - b * per_row) * kSeqKeys;
-  const int64_t len = seq_len(a, b);
-  const int64_t start = a.out_len - len;
-  const bool packed = a.key_offsets != nullptr;
-  int64_t base = b * a.out_len, cap = a.out_len;
-  if (packed) {
-    base = a.key_offsets[b];
-    cap = a.key_offsets[b + 1] - base;
-    cap = cap < 0 ? 0 : (cap > a.out_len ? a.out_len : cap);
-  }
-  for (int j = threadIdx.x; j < kSeqKeys; j += 256) {
-    const int64_t rel = kb + j;
-    if (rel >= cap) break;
-    const bool in_window = rel < len;
-    const int64_t id = in_window ? a.ids[b * a.in_len + seq_src(a, len, rel)] : 0;
-    const bool valid = in_window && (uint64_t)id < (uint64_t)a.f.num_rows && id != a.f.padding_idx;
-    a.keys[base + rel] = valid ? (uint32_t)(a.f.row_base + id) : a.sentinel;
-    a.payload[base + rel] = valid ? (uint32_t)(a.f.payload_base + b * a.out_len + start + rel) : 0u;
-  }
 }
 
 struct LaunchSequence {
@@ -1266,12 +1263,6 @@ int mdl_sequence_forward(const mdl_feature* feature, const int64_t* ids, const i
     const int v = variant_of(d.wdtype, d.odtype, vec, d.dim);
     const int rc = for_each_class(1u << v, LaunchSequence{a, blocks, v % kWidths, s});
     if (rc != MDL_OK) return rc;
-  }
-  if (sort_keys != nullptr && batch > 0 && out_len > 0) {
-    const int64_t blocks = batch * ((out_len + kSeqKeys - 1) / kSeqKeys);
-    if (blocks > 0x7fffffff) return fail(MDL_ERR_UNSUPPORTED, "mdl_sequence_forward: too many positions");
-    hipLaunchKernelGGL(sequence_keys_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);
-    MDL_CHECK_LAUNCH("sequence_keys_kernel");
   }
   return MDL_OK;
 }
