@@ -273,6 +273,14 @@ int mdl_forward(const mdl_feature* feats, int32_t num_features,
                 void* stream);
 
 /*
+ * *mismatched += pooled features of the device array feats whose bag lengths
+ * (offsets, the scan of them) do not add up to their num_ids: the check of
+ * src/model.py:529-551 over every bag of a call at once.
+ */
+int mdl_check_bag_totals(const mdl_feature* feats, int32_t num_features, const int64_t* offsets,
+                         int32_t* mismatched, void* stream);
+
+/*
  * Backward of bag pooling with respect to the pooled rows (the autograd of
  * src/model.py:564-570 and :672-676): for every id position i of a pooled
  * feature, in bag b,

@@ -877,6 +877,15 @@ __global__ __launch_bounds__(kFwdWaves * kWave) void pool_backward_kernel(FwdArg
   with_width<TW, kVec>(v % kWidths, [&]<int C>() { unpool_chunk<TW, TO, C>(f, first, count, s_off[w], a); });
 }
 
+// Pooled features whose bag lengths do not add up to their id count.
+__global__ void bag_totals_kernel(const mdl_feature* __restrict__ feats, int32_t F,
+                                  const int64_t* __restrict__ offsets, int32_t* mismatched) {
+  const int32_t f = blockIdx.x * blockDim.x + threadIdx.x;
+  if (f >= F || feats[f].pooling == MDL_POOL_NONE) return;
+  if (offsets[feats[f].bag_base + feats[f].num_bags] - offsets[feats[f].bag_base] != feats[f].num_ids)
+    atomicAdd(mismatched, 1);
+}
+
 struct LaunchForward {
   const FwdArgs& a;
   int64_t blocks;
@@ -1182,6 +1191,17 @@ int mdl_forward(const mdl_feature* feats, int32_t num_features, const mdl_chunk*
   const int64_t blocks = (num_chunks + kFwdWaves - 1) / kFwdWaves;
   if (blocks > 0x7fffffff) return fail(MDL_ERR_UNSUPPORTED, "mdl_forward: too many chunks");
   return for_each_class(classes, LaunchForward{a, blocks, as_stream(stream), false});
+}
+
+int mdl_check_bag_totals(const mdl_feature* feats, int32_t num_features, const int64_t* offsets, int32_t* mismatched,
+                         void* stream) {
+  if (num_features < 0) return fail(MDL_ERR_INVALID, "mdl_check_bag_totals: negative count");
+  if (num_features == 0) return MDL_OK;
+  if (!feats || !offsets || !mismatched) return fail(MDL_ERR_INVALID, "mdl_check_bag_totals: null pointer");
+  hipLaunchKernelGGL(bag_totals_kernel, dim3((unsigned)((num_features + 255) / 256)), dim3(256), 0, as_stream(stream),
+                     feats, num_features, offsets, mismatched);
+  MDL_CHECK_LAUNCH("bag_totals_kernel");
+  return MDL_OK;
 }
 
 int mdl_pool_backward(const mdl_feature* feats, int32_t num_features, const mdl_chunk* chunks,

@@ -1665,6 +1665,182 @@ Tensor lengths_to_offsets_cuda(const Tensor& lengths_in) {
   return offsets;
 }
 
+// ------------------------------------------------------- bags of rows --
+//
+// Pooling of already-embedded rows (mdl_amd/pooling.py): every flat bag
+// tensor of a call in one lookup launch over features whose rows go by
+// position, and one launch for all their gradients.
+
+// Descriptors of the call's bags; codes[f]: bit 0 null policy "exclude", bit
+// 1 bf16 rows.
+std::vector<mdl_feature> bag_features(at::IntArrayRef rows, at::IntArrayRef dims, at::IntArrayRef batches,
+                                      at::IntArrayRef codes, bool mean) {
+  std::vector<mdl_feature> feats(rows.size(), mdl_feature{});
+  int64_t ids = 0, bags = 0;
+  for (size_t f = 0; f < rows.size(); ++f) {
+    mdl_feature& d = feats[f];
+    d.num_rows = rows[f];
+    d.dim = (int32_t)dims[f];
+    d.wdtype = d.odtype = codes[f] & 2 ? MDL_BF16 : MDL_F32;
+    d.pooling = mean ? MDL_POOL_MEAN : MDL_POOL_SUM;
+    d.flags = MDL_FLAG_ROWS_BY_POSITION | (codes[f] & 1 ? MDL_FLAG_EXCLUDE_NULL : 0);
+    d.table = (int32_t)f;
+    d.payload_base = d.bag_base = bags;
+    d.ids_begin = ids;
+    d.num_ids = rows[f];
+    d.num_bags = batches[f];
+    ids += rows[f];
+    bags += batches[f];
+  }
+  TORCH_CHECK_VALUE(bags < kKeySpace, "a grouped lookup supports fewer than 2^32 - 1 output rows");
+  return feats;
+}
+
+// Chunks of the descriptors, uploaded with them: (device bytes, chunk count).
+std::pair<Tensor, int64_t> upload_chunks(const std::vector<mdl_feature>& feats, int64_t n, const at::Device& dev) {
+  const int F = (int)feats.size();
+  const int target = forward_target_ids(n);
+  const int64_t n_chunks = mdl_plan_chunks(feats.data(), F, target, nullptr, 0);
+  if (n_chunks < 0) check((int)n_chunks, "mdl_plan_chunks");
+  const size_t fbytes = feats.size() * sizeof(mdl_feature);
+  std::vector<uint8_t> host(fbytes + std::max<int64_t>(n_chunks, 1) * sizeof(mdl_chunk));
+  std::memcpy(host.data(), feats.data(), fbytes);
+  if (n_chunks > 0)
+    mdl_plan_chunks(feats.data(), F, target, reinterpret_cast<mdl_chunk*>(host.data() + fbytes), n_chunks);
+  return {upload(host.data(), host.size(), dev), n_chunks};
+}
+
+// (pooled outputs, packed ids, offsets, bag counts).  Without `counter` the
+// reference's errors are raised after one host read; with it (deferred
+// checks) the errors are added to it on the device.
+std::tuple<std::vector<Tensor>, Tensor, Tensor, Tensor> pool_bags_forward(TensorList embedded, TensorList ids,
+                                                                          TensorList lengths, at::IntArrayRef codes,
+                                                                          bool mean,
+                                                                          const std::optional<Tensor>& counter) {
+  const size_t F = embedded.size();
+  TORCH_CHECK_VALUE(F > 0 && ids.size() == F && lengths.size() == F && codes.size() == F,
+                    "one ids, lengths and code entry per bag tensor");
+  const at::Device dev = embedded[0].device();
+  std::vector<int64_t> rows(F), dims(F), batches(F);
+  std::vector<Tensor> len_parts(F);
+  int64_t n = 0, nb = 0;
+  for (size_t f = 0; f < F; ++f) {
+    const Tensor& e = embedded[f];
+    TORCH_CHECK_VALUE(e.dim() == 2 && e.stride(1) == 1 && e.stride(0) == e.size(1),
+                      "embedding weights must be contiguous [rows, dim] tensors");
+    TORCH_CHECK((dtype_code(e.scalar_type()) == MDL_BF16) == ((codes[f] & 2) != 0), "bag code of another dtype");
+    require_device(e, "embedding weight");
+    TORCH_CHECK_VALUE(e.size(0) < kKeySpace, "a table of a grouped lookup holds fewer than 2^32 - 1 rows");
+    TORCH_CHECK_TYPE(ids[f].scalar_type() == at::kLong, "sharded embedding indices must be torch.long");
+    require_device(ids[f], "ids");
+    TORCH_CHECK_VALUE(lengths[f].dim() == 1, "categorical bag lengths must have shape [B]");
+    require_device(lengths[f], "lengths");
+    TORCH_CHECK_VALUE(e.device() == dev && ids[f].device() == dev && lengths[f].device() == dev,
+                      "every bag of a call lives on one device");
+    TORCH_CHECK_VALUE(ids[f].numel() == e.size(0), "categorical bag flat values and embeddings are misaligned");
+    rows[f] = e.size(0);
+    dims[f] = e.size(1);
+    batches[f] = lengths[f].numel();
+    n += rows[f];
+    nb += batches[f];
+    len_parts[f] = lengths[f].scalar_type() == at::kLong ? lengths[f] : lengths[f].to(at::kLong);
+  }
+  const c10::DeviceGuard guard(dev);
+  void* s = stream_of(dev);
+  Tensor all_ids = F == 1 ? ids[0].contiguous() : at::cat(ids).contiguous();
+  if (n == 0) all_ids = at::zeros({1}, all_ids.options());  // any valid address; nothing is read
+  Tensor len_all = (F == 1 ? len_parts[0] : at::cat(len_parts)).contiguous();
+  Tensor offsets = at::empty({nb + 1}, len_all.options());
+  Tensor ws = workspace(mdl_offsets_workspace_bytes(nb), dev);
+  check(mdl_lengths_to_offsets(len_all.data_ptr<int64_t>(), nb, offsets.data_ptr<int64_t>(), ws.data_ptr(),
+                               (size_t)ws.numel(), s),
+        "mdl_lengths_to_offsets");
+  std::vector<mdl_feature> feats = bag_features(rows, dims, batches, codes, mean);
+  std::vector<Tensor> outputs(F);
+  for (size_t f = 0; f < F; ++f) {
+    const int64_t shape[2] = {batches[f], dims[f]};
+    outputs[f] = Tensor(at::detail::empty_cuda(shape, embedded[f].scalar_type(), dev, std::nullopt));
+    feats[f].weight = addr(embedded[f]);
+    feats[f].out = addr(outputs[f]);
+    feats[f].out_stride = dims[f];
+  }
+  auto [meta, n_chunks] = upload_chunks(feats, n, dev);
+  const auto* fd = reinterpret_cast<const mdl_feature*>(meta.data_ptr());
+  const auto* cd = reinterpret_cast<const mdl_chunk*>(static_cast<uint8_t*>(meta.data_ptr()) + F * sizeof(mdl_feature));
+  Tensor bag_count = at::empty({std::max<int64_t>(nb, 1)}, at::TensorOptions().dtype(at::kFloat).device(dev));
+  const bool deferred = counter.has_value() && counter->defined();
+  // errors of the lookup, then features whose lengths do not add up
+  Tensor err = deferred ? *counter : at::zeros({2}, at::TensorOptions().dtype(at::kInt).device(dev));
+  int32_t* ep = err.data_ptr<int32_t>();
+  check(mdl_forward(fd, (int32_t)F, cd, n_chunks, all_ids.data_ptr<int64_t>(), n, offsets.data_ptr<int64_t>(), nullptr,
+                    nullptr, nullptr, 0, bag_count.data_ptr<float>(), ep, mdl_feature_classes(feats.data(), (int32_t)F),
+                    s),
+        "mdl_forward");
+  check(mdl_check_bag_totals(fd, (int32_t)F, offsets.data_ptr<int64_t>(), deferred ? ep : ep + 1, s),
+        "mdl_check_bag_totals");
+  if (!deferred) {
+    const Tensor h = err.to(at::kCPU);
+    const int32_t* bad = h.data_ptr<int32_t>();
+    if (bad[1]) {
+      const Tensor oh = offsets.to(at::kCPU);
+      const int64_t* o = oh.data_ptr<int64_t>();
+      for (size_t f = 0; f < F; ++f) {
+        const int64_t total = o[feats[f].bag_base + batches[f]] - o[feats[f].bag_base];
+        TORCH_CHECK_VALUE(total == rows[f], "categorical bag flat length ", rows[f], " != sum(lengths) ", total);
+      }
+    }
+    TORCH_CHECK_VALUE(bad[0] == 0, "categorical bag lengths must be non-negative");
+  }
+  return {outputs, all_ids, offsets, bag_count};
+}
+
+// The gradient of every bag tensor f with needs[f], in their order, from the
+// pooled outputs' gradients.
+std::vector<Tensor> pool_bags_backward(TensorList grads, at::IntArrayRef needs, at::IntArrayRef rows,
+                                       at::IntArrayRef dims, at::IntArrayRef batches, at::IntArrayRef codes, bool mean,
+                                       const Tensor& ids, const Tensor& offsets, const Tensor& bag_count) {
+  const size_t F = grads.size();
+  TORCH_CHECK_VALUE(needs.size() == F && rows.size() == F && dims.size() == F && batches.size() == F &&
+                        codes.size() == F,
+                    "one entry per bag tensor");
+  const at::Device dev = ids.device();
+  const c10::DeviceGuard guard(dev);
+  const std::vector<mdl_feature> all = bag_features(rows, dims, batches, codes, mean);
+  std::vector<mdl_feature> feats;
+  std::vector<Tensor> dests, keep;
+  int64_t n = 0, n_all = 0;
+  for (size_t f = 0; f < F; ++f) {
+    n_all += rows[f];
+    if (!needs[f]) continue;
+    const auto dtype = codes[f] & 2 ? at::kBFloat16 : at::kFloat;
+    Tensor g = grads[f];
+    require_device(g, "gradient");
+    TORCH_CHECK_VALUE(g.numel() == batches[f] * dims[f], "the gradient of a pooled output has its shape");
+    if (g.scalar_type() != dtype) g = g.to(dtype);
+    if (g.dim() != 2 || g.stride(-1) != 1) g = g.reshape({-1, dims[f]}).contiguous();
+    const int64_t shape[2] = {rows[f], dims[f]};
+    Tensor d = Tensor(at::detail::empty_cuda(shape, dtype, dev, std::nullopt));
+    mdl_feature rec = all[f];
+    rec.out = addr(g);
+    rec.out_stride = g.stride(0);
+    rec.weight = addr(d);
+    feats.push_back(rec);
+    keep.push_back(std::move(g));
+    dests.push_back(std::move(d));
+    n += rows[f];
+  }
+  if (feats.empty()) return dests;
+  auto [meta, n_chunks] = upload_chunks(feats, n, dev);
+  check(mdl_pool_backward(reinterpret_cast<const mdl_feature*>(meta.data_ptr()), (int32_t)feats.size(),
+                          reinterpret_cast<const mdl_chunk*>(static_cast<uint8_t*>(meta.data_ptr()) +
+                                                             feats.size() * sizeof(mdl_feature)),
+                          n_chunks, ids.data_ptr<int64_t>(), n_all, offsets.data_ptr<int64_t>(),
+                          bag_count.data_ptr<float>(), mdl_feature_classes(feats.data(), (int32_t)feats.size()),
+                          stream_of(dev)),
+        "mdl_pool_backward");
+  return dests;
+}
+
 // ------------------------------------------------------------- sequences --
 
 mdl_feature sequence_record(const Tensor& weight, int64_t padding_idx) {
@@ -1920,6 +2096,13 @@ TORCH_LIBRARY(mdl_hip, m) {
         "Tensor payload, int num_entries, Tensor? bag_count, Tensor(a!) sumsq, int slot, Tensor(b!) workspace, "
         "int max_dim, int key_bits, int classes) -> ()",
         &backward_sumsq_);
+  // Pooling of already-embedded rows (mdl_amd/pooling.py's autograd function).
+  m.def("pool_bags_forward(Tensor[] embedded, Tensor[] ids, Tensor[] lengths, int[] codes, bool mean, "
+        "Tensor(a!)? counter) -> (Tensor[], Tensor, Tensor, Tensor)",
+        &pool_bags_forward);
+  m.def("pool_bags_backward(Tensor[] grads, int[] needs, int[] rows, int[] dims, int[] batches, int[] codes, "
+        "bool mean, Tensor ids, Tensor offsets, Tensor bag_count) -> Tensor[]",
+        &pool_bags_backward);
   m.def("clip_coefficient_(Tensor sumsq, int count, float max_norm, Tensor(a!) total_norm, Tensor(b!) coef) -> ()",
         &clip_coefficient_);
   // The trainer's sparse clip over parameter lists (their gradients scaled

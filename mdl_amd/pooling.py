@@ -25,11 +25,10 @@ from __future__ import annotations
 
 from typing import Sequence
 
-import numpy as np
 import torch
 from torch import Tensor
 
-from . import ops
+from . import library, ops  # noqa: F401  (library registers the mdl_hip ops)
 from .embeddings import _deferred_counter, deferred_index_checks
 
 _POLICIES = ("exclude", "include_as_padding")
@@ -74,53 +73,31 @@ def _as_flat(
 
 
 class _BagPoolFn(torch.autograd.Function):
+    """One ``mdl_hip::pool_bags_forward`` call over every bag tensor, and one
+    ``pool_bags_backward`` call for their gradients (descriptors, chunk plans
+    and the length checks in C++)."""
+
     @staticmethod
     def forward(ctx, ctl: dict, *embedded: Tensor):  # type: ignore[override]
-        plan: ops.GroupPlan = ctl["plan"]
-        res = ops.grouped_forward(
-            plan, ctl["ids"], ctl["lengths"], with_backward=False, with_bag_count=True,
-            error_count=ctl["error_count"],
+        codes = ctl["codes"]
+        pooled, ids, offsets, bag_count = torch.ops.mdl_hip.pool_bags_forward(
+            list(embedded), ctl["ids"], ctl["lengths"], codes, ctl["mean"], ctl["counter"],
         )
-        _check_lengths(res, ctl)
-        ctx.res = res
+        ctx.saved = (codes, ctl["mean"], ids, offsets, bag_count)
         ctx.rows = [int(e.size(0)) for e in embedded]
-        return tuple(res.outputs)
+        ctx.dims = [int(e.size(1)) for e in embedded]
+        ctx.batches = [int(p.size(0)) for p in pooled]
+        return tuple(pooled)
 
     @staticmethod
     def backward(ctx, *grads: Tensor):  # type: ignore[override]
-        res: ops.ForwardResult = ctx.res
-        dests: list[Tensor | None] = []
-        for f, spec in enumerate(res.plan.features):
-            if not ctx.needs_input_grad[1 + f]:
-                dests.append(None)
-                continue
-            w = res.plan.tables[spec.table].weight
-            dests.append(torch.empty((ctx.rows[f], int(w.size(1))), dtype=w.dtype, device=w.device))
-        ops.pool_backward(res, list(grads), dests)
-        ctx.res = None
-        return (None, *dests)
-
-
-def _check_lengths(res: ops.ForwardResult, ctl: dict) -> None:
-    """sum(lengths) must equal the flat length of every bag (src/model.py:529-551)."""
-
-    feats = res.feats
-    if len(feats) == 0:
-        return
-    host = np.stack([feats["bag_base"], feats["bag_base"] + feats["num_bags"], feats["num_ids"]]).astype(np.int64)
-    starts, ends, counts = ops.upload(host, res.device).view(torch.int64).view(3, -1)
-    mismatched = (res.offsets[ends] - res.offsets[starts]).ne(counts).sum(dtype=torch.int32)
-    if ctl["deferred"]:
-        res.error_count.add_(mismatched)
-        return
-    bad = torch.stack([mismatched, res.error_count.reshape(())]).tolist()
-    if bad[0]:
-        sums = (res.offsets[ends] - res.offsets[starts]).tolist()
-        for n, total in zip(feats["num_ids"].tolist(), sums):
-            if n != total:
-                raise ValueError(f"categorical bag flat length {n} != sum(lengths) {total}")
-    if bad[1]:
-        raise ValueError("categorical bag lengths must be non-negative")
+        codes, mean, ids, offsets, bag_count = ctx.saved
+        needs = [int(n) for n in ctx.needs_input_grad[1:]]
+        got = iter(torch.ops.mdl_hip.pool_bags_backward(
+            list(grads), needs, ctx.rows, ctx.dims, ctx.batches, codes, mean, ids, offsets, bag_count,
+        ))
+        ctx.saved = None
+        return (None, *(next(got) if n else None for n in needs))
 
 
 def pool_bags(
@@ -135,7 +112,7 @@ def pool_bags(
     if mode not in ("mean", "sum"):
         raise ValueError(f"unsupported pooling {mode!r}")
     outputs: list[Tensor | None] = [None] * len(items)
-    plan = ops.GroupPlan()
+    codes: list[int] = []
     ids: list[Tensor] = []
     lengths: list[Tensor] = []
     inputs: list[Tensor] = []
@@ -148,19 +125,18 @@ def pool_bags(
         if idx.dtype != torch.long:
             idx = idx.long()
         emb = ops._row_major_aligned(emb)
-        plan.add_feature(emb, pooling=mode, null_policy=pol, padding_idx=0, rows_by_position=True)
+        codes.append((1 if pol == "exclude" else 0) | (2 if ops.dtype_code(emb.dtype) == ops.MDL_BF16 else 0))
         ids.append(idx.contiguous())
         lengths.append(ln)
         inputs.append(emb)
         slots.append((k, padded))
     if inputs:
-        deferred = deferred_index_checks()
         ctl = {
-            "plan": plan,
+            "codes": codes,
+            "mean": mode == "mean",
             "ids": ids,
             "lengths": lengths,
-            "deferred": deferred,
-            "error_count": _deferred_counter(inputs[0].device) if deferred else None,
+            "counter": _deferred_counter(inputs[0].device) if deferred_index_checks() else None,
         }
         pooled = _BagPoolFn.apply(ctl, *inputs)
         for (k, _), out in zip(slots, pooled):
