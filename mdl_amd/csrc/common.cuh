@@ -72,6 +72,8 @@ struct BagDivisor {
     r = kBagRcp.v[i < kRcpTable ? i : 0];
     if (__builtin_expect(i >= kRcpTable, 0)) r = bag_rcp_slow(count);
   }
+  // (count, reciprocal) of a divisor made before
+  __device__ __forceinline__ explicit BagDivisor(float2 made) : d(made.x), r(made.y) {}
   __device__ __forceinline__ float operator()(float v) const {
     const float q = __fmul_rn(v, r);
     return __builtin_fmaf(__builtin_fmaf(-q, d, v), r, q);

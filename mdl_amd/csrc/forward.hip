@@ -792,76 +792,108 @@ __global__ MDL_OCCUPANCY __launch_bounds__(kFwdWaves * kWave) void forward_kerne
 
 // ------------------------------------------------------ pool backward --
 
+// Per-wave LDS of an unpooled chunk: bag bounds relative to the chunk's first
+// position, every bag's divisor with its reciprocal, and the bag of each
+// position of one window (kNoBag: the position's gradient is zero).
+constexpr int kPosWindow = 512;
+constexpr uint16_t kNoBag = 0xffff;
+struct UnpoolStage {
+  int64_t off[kMaxBagsPerChunk + 1];
+  float2 div[kMaxBagsPerChunk];
+  uint16_t bag[kPosWindow];
+};
+
 // Per-position gradient of one chunk of bags: slot e of bag b receives the
 // bag's upstream gradient row times w_e / max(count_b, 1) (mean) or w_e (sum).
-// The walk over the chunk's positions visits consecutive slots of one bag
-// together, so they read the same gradient row, which stays in L2: HBM sees
-// about one read of each pooled gradient row and one write of each position
-// row.
+// The positions' bags and null weights are staged first, one position per
+// lane, with the bags' divisors, so the walk is gradient rows in (each read
+// by its bag's consecutive positions, from L2) and position rows out.  Found
+// and divided in the walk, id by id, the launch took 51 us for 8 fp32 bag
+// tensors of 67584 x 32-64 (104 MB written); staged, 30.5 us.
 template <typename TW, typename TO, int C>
-__device__ __forceinline__ void unpool_chunk(const Feat& f, int64_t first_bag, int nb, int64_t* s_off,
+__device__ __forceinline__ void unpool_chunk(const Feat& f, int64_t first_bag, int nb, UnpoolStage& st,
                                              const FwdArgs& a) {
-  constexpr int kUnroll = unroll_for<C>();
+  constexpr int kUnroll = C == 1 ? 4 : (32 / C > 1 ? 32 / C : 1);
+  constexpr bool kSplit = MDL_SPLIT_ROWS && std::is_same_v<TW, float> && std::is_same_v<TO, float> && C == 8;
   const int lane = lane_id();
-  stage_offsets(f, first_bag, nb, s_off, a);
-  const int64_t e_begin = s_off[0], e_end = s_off[nb];
+  const bool mean = f.pooling == MDL_POOL_MEAN;
+  const float* counts = a.bag_count + f.payload_base + first_bag;
+  for (int i = lane; i < nb; i += kWave) {
+    // grad / max(count, 1): the autograd of the reference's division
+    const BagDivisor d(mean ? fmaxf(ld_policy(counts + i), 1.f) : 1.f);
+    st.div[i] = make_float2(d.d, d.r);
+  }
+  stage_offsets(f, first_bag, nb, st.off, a);
+  const int64_t e_begin = st.off[0], e_end = st.off[nb];
   const int L = lanes_for(f.dim, C);
   const int G = kWave / L;
   const int slot = lane / L, sub = lane % L;
   const int ncb = (f.dim + L * C - 1) / (L * C);
   const bool exclude = (f.flags & MDL_FLAG_EXCLUDE_NULL) != 0;
   const bool by_pos = (f.flags & MDL_FLAG_ROWS_BY_POSITION) != 0;
-  const bool mean = f.pooling == MDL_POOL_MEAN;
   const TO* grad = static_cast<const TO*>(f.out);
   TW* dst = static_cast<TW*>(const_cast<void*>(f.weight));
-  const float* counts = a.bag_count + f.payload_base + first_bag;
-  const int64_t step = (int64_t)G * kUnroll;
-  for (int cb = 0; cb < ncb; ++cb) {
-    const int col = (cb * L + sub) * C;
-    const bool col_ok = col < f.dim;
-    int bag = 0;
-    for (int64_t base = e_begin; base < e_end; base += step) {
-      int64_t id[kUnroll];
-      int bg[kUnroll];
-      bool valid[kUnroll];
-      float cnt[kUnroll], v[kUnroll][C];
+  const int step = G * kUnroll;
+  for (int64_t w0 = e_begin; w0 < e_end; w0 += kPosWindow) {
+    const int wn = e_end - w0 < kPosWindow ? (int)(e_end - w0) : kPosWindow;
+    constexpr int kBatch = 4;
+    for (int i0 = lane; i0 < wn; i0 += kWave * kBatch) {
+      int64_t id[kBatch];
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        const int64_t e = base + (int64_t)u * G + slot;
-        valid[u] = e < e_end;
-        id[u] = valid[u] ? a.ids[e] : 0;
-        if (valid[u]) {
-          while (s_off[bag + 1] <= e) ++bag;
-        }
-        bg[u] = bag;
-      }
+      for (int q = 0; q < kBatch; ++q) id[q] = i0 + q * kWave < wn ? ld_policy(a.ids + w0 + i0 + q * kWave) : 0;
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        cnt[u] = *(mean && valid[u] ? counts + bg[u] : zero_row<float>());
-        RowIO<TO, C>::load(valid[u] && col_ok ? grad + (first_bag + bg[u]) * f.out_stride + col : zero_row<TO>(),
-                           v[u]);
-      }
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        const int64_t e = base + (int64_t)u * G + slot;
-        const int64_t row = e - f.ids_begin;
+      for (int q = 0; q < kBatch; ++q) {
+        const int i = i0 + q * kWave;
+        if (i >= wn) break;
         // Positions the forward gave weight 0: nulls under "exclude" and rows
         // outside [0, num_rows).
-        const int64_t src = by_pos ? row : id[u];
-        const bool dead = (exclude && id[u] == 0) || (uint64_t)src >= (uint64_t)f.num_rows;
-        // grad / max(count, 1): the autograd of the reference's division
-        const BagDivisor div(mean ? fmaxf(cnt[u], 1.f) : 1.f);
-#pragma unroll
-        for (int k = 0; k < C; ++k) v[u][k] = dead ? 0.f : div(v[u][k]);
-        if (valid[u] && col_ok) RowIO<TW, C>::store(dst + row * f.dim + col, v[u]);
+        const int64_t src = by_pos ? w0 + i - f.ids_begin : id[q];
+        const bool dead = (exclude && id[q] == 0) || (uint64_t)src >= (uint64_t)f.num_rows;
+        st.bag[i] = dead ? kNoBag : (uint16_t)bag_of(st.off, nb, w0 + i);
       }
     }
+    wave_sync();
+    TW* rows = dst + (w0 - f.ids_begin) * f.dim;
+    for (int cb = 0; cb < ncb; ++cb) {
+      // (split rows: two 16-byte pieces 4L elements apart, as the lookup's)
+      const int col = kSplit ? cb * L * C + sub * 4 : (cb * L + sub) * C;
+      const bool col_ok = col < f.dim;
+      const int pieces = col + 4 * L < f.dim ? 2 : 1;
+      for (int base = 0; base < wn; base += step) {
+        float v[kUnroll][C];
+        float2 div[kUnroll];
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+          const int i = base + u * G + slot;
+          const uint16_t bag = i < wn ? st.bag[i] : kNoBag;
+          const bool live = bag != kNoBag && col_ok;
+          div[u] = st.div[bag != kNoBag ? bag : 0];
+          const TO* g = live ? grad + (first_bag + bag) * f.out_stride + col : zero_row<TO>();
+          if constexpr (kSplit) RowIO<float, C>::load_pieces(g, 4 * L, live ? pieces : 0, v[u]);
+          else RowIO<TO, C>::load(g, v[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+          const int i = base + u * G + slot;
+          const BagDivisor d(div[u]);
+#pragma unroll
+          for (int k = 0; k < C; ++k) v[u][k] = d(v[u][k]);
+          if (i < wn && col_ok) {
+            if constexpr (kSplit)
+              RowIO<float, C>::template store_pieces<kOutPolicy>(rows + (int64_t)i * f.dim + col, 4 * L, pieces, v[u]);
+            else
+              RowIO<TW, C>::template store<kOutPolicy>(rows + (int64_t)i * f.dim + col, v[u]);
+          }
+        }
+      }
+    }
+    wave_sync();  // the next window restages the bags
   }
 }
 
 template <typename TW, typename TO, bool kVec>
-__global__ __launch_bounds__(kFwdWaves * kWave) void pool_backward_kernel(FwdArgs a) {
-  __shared__ int64_t s_off[kFwdWaves][kMaxBagsPerChunk + 1];
+__global__ MDL_OCCUPANCY __launch_bounds__(kFwdWaves * kWave) void pool_backward_kernel(FwdArgs a) {
+  __shared__ UnpoolStage s_st[kFwdWaves];
   const int w = threadIdx.x / kWave;
   const int64_t blk = xcd_block(blockIdx.x, gridDim.x);
   const int64_t c = uni64(blk * kFwdWaves + w);
@@ -874,7 +906,7 @@ __global__ __launch_bounds__(kFwdWaves * kWave) void pool_backward_kernel(FwdArg
   if (v / kWidths != ClassOf<TW, TO, kVec>::value) return;  // another class's launch owns it
   if (f.pooling == MDL_POOL_NONE || count > kMaxBagsPerChunk || count <= 0) return;
   bind_range(f, a);
-  with_width<TW, kVec>(v % kWidths, [&]<int C>() { unpool_chunk<TW, TO, C>(f, first, count, s_off[w], a); });
+  with_width<TW, kVec>(v % kWidths, [&]<int C>() { unpool_chunk<TW, TO, C>(f, first, count, s_st[w], a); });
 }
 
 // Pooled features whose bag lengths do not add up to their id count.
