@@ -364,17 +364,75 @@ __global__ __launch_bounds__(256) void count_heads_kernel(const int64_t* __restr
   if (lane == 0) heads[c] = cnt;
 }
 
+// Distinct-row range of table t from the scanned head counts.
+__device__ __forceinline__ void write_unique_range(int32_t t, const int64_t* table_start, const int64_t* table_end,
+                                                   const int64_t* chunk_base, const int64_t* head_base,
+                                                   const mdl_table* __restrict__ tables, int64_t* unique_range,
+                                                   ChunkRule rule) {
+  const int64_t lo = table_start[t], hi = table_end[t];
+  const int64_t cb = table_chunk_len(tables[t], rule);
+  const int64_t nch = (hi - lo + cb - 1) / cb;
+  unique_range[2 * t] = head_base[chunk_base[t]];
+  unique_range[2 * t + 1] = head_base[chunk_base[t] + nch];
+}
+
 __global__ void unique_range_end_kernel(int32_t T, const int64_t* table_start, const int64_t* table_end,
                                         const int64_t* chunk_base, const int64_t* head_base,
                                         const mdl_table* __restrict__ tables, int64_t* unique_range,
                                         ChunkRule rule) {
-  for (int32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < T; t += gridDim.x * blockDim.x) {
-    const int64_t lo = table_start[t], hi = table_end[t];
-    const int64_t cb = table_chunk_len(tables[t], rule);
-    const int64_t nch = (hi - lo + cb - 1) / cb;
-    unique_range[2 * t] = head_base[chunk_base[t]];
-    unique_range[2 * t + 1] = head_base[chunk_base[t] + nch];
+  for (int32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < T; t += gridDim.x * blockDim.x)
+    write_unique_range(t, table_start, table_end, chunk_base, head_base, tables, unique_range, rule);
+}
+
+// The scan of the chunks' head counts and the tables' ranges in one block:
+// calls of few chunks would spend a launch on each (two for the scan).
+constexpr int kHeadThreads = 1024;
+constexpr int kHeadItems = 8;
+constexpr int64_t kHeadBlockChunks = 4 * kHeadThreads * kHeadItems;
+
+__global__ __launch_bounds__(kHeadThreads) void heads_range_kernel(
+    const int64_t* __restrict__ heads, const int64_t* __restrict__ num_chunks, int64_t max_chunks, int32_t T,
+    const int64_t* table_start, const int64_t* table_end, const int64_t* chunk_base, int64_t* head_base,
+    const mdl_table* __restrict__ tables, int64_t* unique_range, ChunkRule rule) {
+  __shared__ int32_t s_wave[kHeadThreads / kWave];
+  const int64_t m = *num_chunks < max_chunks ? *num_chunks : max_chunks;
+  const int tid = threadIdx.x, w = tid / kWave, lane = lane_id();
+  int64_t carry = 0;
+  if (tid == 0) head_base[0] = 0;
+  for (int64_t base = 0; base < m; base += kHeadThreads * kHeadItems) {
+    const int64_t first = base + (int64_t)tid * kHeadItems;
+    int32_t v[kHeadItems], s = 0;  // (a chunk has at most 512 heads)
+#pragma unroll
+    for (int k = 0; k < kHeadItems; ++k) v[k] = first + k < m ? (int32_t)heads[first + k] : 0;
+#pragma unroll
+    for (int k = 0; k < kHeadItems; ++k) s += v[k];
+    int32_t x = s;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const int o = shfl_i(x, lane >= d ? lane - d : lane);
+      if (lane >= d) x += o;
+    }
+    if (lane == kWave - 1) s_wave[w] = x;
+    __syncthreads();
+    int32_t before = 0, all = 0;
+#pragma unroll
+    for (int q = 0; q < kHeadThreads / kWave; ++q) {
+      before += q < w ? s_wave[q] : 0;
+      all += s_wave[q];
+    }
+    int64_t run = carry + before + x - s;
+#pragma unroll
+    for (int k = 0; k < kHeadItems; ++k) {
+      run += v[k];
+      if (first + k < m) head_base[first + k + 1] = run;
+    }
+    carry += all;
+    __syncthreads();  // (also: this block's head_base writes before the reads below)
   }
+  __threadfence_block();
+  __syncthreads();
+  for (int32_t t = tid; t < T; t += kHeadThreads)
+    write_unique_range(t, table_start, table_end, chunk_base, head_base, tables, unique_range, rule);
 }
 
 __global__ void unique_range_zero(int32_t T, int64_t* unique_range) {
@@ -1508,6 +1566,12 @@ int mdl_backward_count_hinted(const mdl_table* tables, int32_t num_tables, int32
   hipLaunchKernelGGL(count_heads_kernel, dim3((unsigned)((mc + 3) / 4)), dim3(256), 0, s, w.num_chunks, w.desc,
                      sk, mc, heads);
   MDL_CHECK_LAUNCH("count_heads_kernel");
+  if (mc <= kHeadBlockChunks) {
+    hipLaunchKernelGGL(heads_range_kernel, dim3(1), dim3(kHeadThreads), 0, s, heads, w.num_chunks, mc, num_tables,
+                       w.table_start, w.table_end, w.chunk_base, w.head_base, tables, unique_range, chunk_rule(n));
+    MDL_CHECK_LAUNCH("heads_range_kernel");
+    return MDL_OK;
+  }
   rc = mdl_lengths_to_offsets(heads, mc, w.head_base, w.scan_ws, w.scan_bytes, stream);
   if (rc) return rc;
   hipLaunchKernelGGL(unique_range_end_kernel, dim3((unsigned)((num_tables + 255) / 256)), dim3(256), 0, s,

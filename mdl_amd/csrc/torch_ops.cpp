@@ -663,7 +663,15 @@ CoalesceResult coalesce_groups(const Layout& L, std::vector<mdl_feature>& feats,
   r.vbuf = at::empty({std::max<int64_t>(lay.val_off[T], 1)}, at::TensorOptions().dtype(at::kByte).device(dev));
   int64_t n_ranges = 0;
   for (const auto& g : L.groups) n_ranges += 2 * (int64_t)g.tables.size();
-  Tensor urange = at::zeros({n_ranges}, at::TensorOptions().dtype(at::kLong).device(dev));
+  // every range of a group with entries is written by its count
+  bool all_groups = true;
+  for (const auto& g : L.groups) {
+    int64_t n = 0;
+    for (int f = g.lo; f < g.hi; ++f) n += feats[f].num_ids;
+    all_groups = all_groups && n > 0;
+  }
+  auto i64 = at::TensorOptions().dtype(at::kLong).device(dev);
+  Tensor urange = all_groups ? at::empty({n_ranges}, i64) : at::zeros({n_ranges}, i64);
   const uint64_t rows_base = addr(r.rows_all), vals_base = addr(r.vbuf);
   struct Launch {
     const mdl_feature* fd;
@@ -723,19 +731,27 @@ CoalesceResult coalesce_groups(const Layout& L, std::vector<mdl_feature>& feats,
           "mdl_backward_count");
     launches.push_back(std::move(l));
   }
-  Tensor diff = urange.slice(0, 1, n_ranges, 2) - urange.slice(0, 0, n_ranges, 2);
-  if (L.groups.size() == 1) {
-    r.counts = diff;
-  } else {
-    std::vector<int64_t> order;
-    for (const auto& g : L.groups)
-      for (int t : g.tables) order.push_back(t);
-    r.counts = at::zeros({T}, urange.options());
-    r.counts.index_copy_(0, upload_vec(order, dev).view(at::kLong).narrow(0, 0, (int64_t)order.size()), diff);
-  }
   if (host_counts) {
-    Tensor h = r.counts.to(at::kCPU);
-    host_counts->assign(h.data_ptr<int64_t>(), h.data_ptr<int64_t>() + T);
+    // the ranges are read as they are and subtracted here
+    const Tensor h = urange.to(at::kCPU);
+    const int64_t* u = h.data_ptr<int64_t>();
+    host_counts->assign(T, 0);
+    for (const auto& g : L.groups)
+      for (int t : g.tables) {
+        (*host_counts)[t] = u[1] - u[0];
+        u += 2;
+      }
+  } else {
+    Tensor diff = urange.slice(0, 1, n_ranges, 2) - urange.slice(0, 0, n_ranges, 2);
+    if (L.groups.size() == 1) {
+      r.counts = diff;
+    } else {
+      std::vector<int64_t> order;
+      for (const auto& g : L.groups)
+        for (int t : g.tables) order.push_back(t);
+      r.counts = at::zeros({T}, urange.options());
+      r.counts.index_copy_(0, upload_vec(order, dev).view(at::kLong).narrow(0, 0, (int64_t)order.size()), diff);
+    }
   }
   for (const Launch& l : launches) {
     check(mdl_backward_coalesce(l.fd, l.nf, l.td, l.Tg, L.max_dim, l.k, l.p, l.n, L.key_bits,
@@ -1898,7 +1914,7 @@ std::tuple<Tensor, Tensor, Tensor> sequence_lookup_backward_cuda(const Tensor& w
                                                                  const Tensor& lengths, int64_t out_len,
                                                                  bool newest_first, int64_t padding_idx,
                                                                  const Tensor& grad, const Tensor& keys_in,
-                                                                 const Tensor& payload_in) {
+                                                                 const Tensor& payload_in, bool pad) {
   require_device(weight, "embedding weight");
   const at::Device dev = weight.device();
   const c10::DeviceGuard guard(dev);
@@ -1919,7 +1935,7 @@ std::tuple<Tensor, Tensor, Tensor> sequence_lookup_backward_cuda(const Tensor& w
   feats[0].grad = addr(g);
   feats[0].out = addr(g);
   feats[0].out_stride = g.stride(0);
-  CoalesceResult r = coalesce_groups(*L, feats, keys, payload, Tensor(), {n}, dev);
+  CoalesceResult r = coalesce_groups(*L, feats, keys, payload, Tensor(), {n}, dev, pad);
   Tensor rows = r.rows_all.narrow(0, 0, n);
   Tensor vals = r.vbuf.narrow(0, 0, r.layout.nbytes[0]).view(weight.scalar_type()).view({n, dim});
   return {rows, vals, r.counts};
@@ -2051,7 +2067,7 @@ TORCH_LIBRARY(mdl_hip, m) {
   m.def("sequence_lookup(Tensor weight, Tensor ids, Tensor lengths, int out_len, bool newest_first, "
         "int padding_idx, bool need_backward) -> (Tensor, Tensor, Tensor, Tensor, Tensor)");
   m.def("sequence_lookup_backward(Tensor weight, Tensor ids, Tensor lengths, int out_len, bool newest_first, "
-        "int padding_idx, Tensor grad, Tensor keys, Tensor payload) -> (Tensor, Tensor, Tensor)");
+        "int padding_idx, Tensor grad, Tensor keys, Tensor payload, bool pad=True) -> (Tensor, Tensor, Tensor)");
   m.def("sparse_coalesce(Tensor indices, Tensor values, int num_rows) -> (Tensor, Tensor)");
   m.def("sparse_coalesce_padded(Tensor indices, Tensor values, int num_rows) -> (Tensor, Tensor, Tensor)");
   m.def("rowwise_adagrad_(Tensor(a!) weight, Tensor(b!) accumulator, Tensor rows, Tensor values, float lr, "

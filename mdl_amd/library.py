@@ -526,7 +526,7 @@ def _sequence_lookup_fake(weight, ids, lengths, out_len, newest_first, padding_i
 
 
 @_cpu_kernel("sequence_lookup_backward")
-def _sequence_backward_cpu(weight, ids, lengths, out_len, newest_first, padding_idx, grad, keys, payload):
+def _sequence_backward_cpu(weight, ids, lengths, out_len, newest_first, padding_idx, grad, keys, payload, pad=True):
     mask, src = _window_cpu(ids, lengths, out_len, newest_first)
     rows = torch.gather(ids, 1, src) if ids.size(1) else torch.zeros_like(src)
     keep = mask & (rows >= 0) & (rows < weight.size(0)) & rows.ne(padding_idx)
@@ -537,7 +537,7 @@ def _sequence_backward_cpu(weight, ids, lengths, out_len, newest_first, padding_
 
 
 @_fake_kernel("sequence_lookup_backward")
-def _sequence_backward_fake(weight, ids, lengths, out_len, newest_first, padding_idx, grad, keys, payload):
+def _sequence_backward_fake(weight, ids, lengths, out_len, newest_first, padding_idx, grad, keys, payload, pad=True):
     n = int(ids.size(0)) * int(out_len)
     return (weight.new_empty(n, dtype=torch.int64), weight.new_empty((n, weight.size(1))),
             weight.new_empty(1, dtype=torch.int64))
@@ -549,6 +549,8 @@ def _sequence_setup(ctx, inputs, output):
     ctx.save_for_backward(weight, ids, lengths, keys, payload)
     ctx.args = (int(out_len), bool(newest_first), int(padding_idx))
     ctx.mark_non_differentiable(mask)
+    # the mask, keys, payloads and count get no gradient: none is made of zeros
+    ctx.set_materialize_grads(False)
 
 
 def _sequence_backward(ctx, grad_out, *_unused):
@@ -556,10 +558,13 @@ def _sequence_backward(ctx, grad_out, *_unused):
     out_len, newest_first, padding_idx = ctx.args
     if grad_out is None:
         grad_out = torch.zeros((ids.size(0), out_len, weight.size(1)), dtype=weight.dtype, device=weight.device)
+    # an exact gradient views the live rows only: nothing past them is filled
+    eager = _eager(keys)
     rows, values, count = torch.ops.mdl_hip.sequence_lookup_backward(
         weight, ids, lengths, out_len, newest_first, padding_idx, grad_out.contiguous(), keys, payload,
+        not (eager and _grad_mode == "coalesced"),
     )
-    if _eager(rows):
+    if eager:
         g = torch.ops.mdl_hip.capacity_sparse_grad(weight, rows, values, count, _grad_mode == "coalesced")
     else:
         g = torch.sparse_coo_tensor(rows.unsqueeze(0), values, tuple(weight.shape), is_coalesced=False)
