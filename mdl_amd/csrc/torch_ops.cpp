@@ -544,7 +544,13 @@ std::tuple<std::vector<Tensor>, Tensor, Tensor, Tensor, Tensor, Tensor> grouped_
     payload = n ? at::empty({n}, i32) : at::zeros({1}, i32);
   }
   Tensor bag_count = at::empty({0}, at::TensorOptions().dtype(at::kFloat).device(dev));
-  if (L->pooled_any) bag_count = at::zeros({std::max<int64_t>(total_rows, 1)}, bag_count.options());
+  if (L->pooled_any) {
+    // the lookup writes every bag's count; rows of unpooled features have none
+    bool all_pooled = n_chunks > 0;
+    for (int f = 0; f < F; ++f) all_pooled = all_pooled && L->feats[f].pooling != MDL_POOL_NONE;
+    const int64_t entries = std::max<int64_t>(total_rows, 1);
+    bag_count = all_pooled ? at::empty({entries}, bag_count.options()) : at::zeros({entries}, bag_count.options());
+  }
   uint8_t* mbase = static_cast<uint8_t*>(meta.data_ptr());
   check(mdl_forward(reinterpret_cast<const mdl_feature*>(mbase), F, reinterpret_cast<const mdl_chunk*>(mbase + fbytes),
                     n_chunks, ids_arg.data_ptr<int64_t>(), n, offsets.defined() ? offsets.data_ptr<int64_t>() : nullptr,
@@ -1102,6 +1108,9 @@ struct GroupedLookupFn : public torch::autograd::Function<GroupedLookupFn> {
     sd["bag_count"] = bag_count;
     sd["offsets"] = offsets;
     ctx->mark_non_differentiable({err});
+    // no zero gradient is made for the error count; an output that the loss
+    // does not reach gets its zeros in the backward
+    ctx->set_materialize_grads(false);
     outputs.push_back(err);
     return outputs;
   }
@@ -1114,8 +1123,19 @@ struct GroupedLookupFn : public torch::autograd::Function<GroupedLookupFn> {
     const std::vector<Tensor> weights = sd["weights"].toTensorVector();
     const std::vector<Tensor> ids = sd["ids"].toTensorVector();
     grads.pop_back();  // err
+    const auto lengths = sd["lengths"].toOptionalTensorList();
+    const auto table = sd["table"].toIntVector(), pooling = sd["pooling"].toIntVector();
+    for (size_t f = 0; f < grads.size(); ++f) {
+      if (grads[f].defined()) continue;
+      const Tensor& w = weights[table[f]];
+      std::vector<int64_t> shape;
+      if (pooling[f] == MDL_POOL_NONE) shape = ids[f].sizes().vec();
+      else shape = {lengths.get(f)->numel()};
+      shape.push_back(w.size(1));
+      grads[f] = at::zeros(shape, w.options());
+    }
     const std::vector<std::optional<Tensor>> wg = weight_grads_for(
-        weights, ids, sd["lengths"].toOptionalTensorList(), sd["table"].toIntVector(), sd["pooling"].toIntVector(),
+        weights, ids, lengths, table, pooling,
         sd["exclude"].toIntVector(), sd["padding_idx"].toIntVector(), grads, sd["keys"].toTensor(),
         sd["payload"].toTensor(), sd["bag_count"].toTensor(), sd["offsets"].toTensor(), g_exact_grads.load(), true);
     torch::autograd::variable_list out(weights.size() + 6);
