@@ -274,9 +274,102 @@ __global__ __launch_bounds__(256) void bwd_desc_kernel(const mdl_table* __restri
   }
 }
 
+// Bounds and chunk plan of a call of few tables in one launch: every block
+// finds all the tables' bounds (a thread each: a search among 256 sampled
+// keys in LDS, then in the stretch between two of them) and writes the
+// descriptors of its own table.  The two kernels above take a launch each,
+// 8.0 us together for 393 K entries of 32 tables; this one takes 7.5 and a
+// launch less of the host.
+__global__ __launch_bounds__(kBoundThreads) void bwd_plan_kernel(const mdl_table* __restrict__ tables, int32_t T,
+                                                                 const uint32_t* __restrict__ keys, int64_t n_cap,
+                                                                 const int64_t* __restrict__ n_dev,
+                                                                 int64_t* __restrict__ table_start,
+                                                                 int64_t* __restrict__ table_end,
+                                                                 int64_t* __restrict__ chunk_base,
+                                                                 int64_t* __restrict__ total,
+                                                                 ChunkDesc* __restrict__ desc, int64_t max_chunks,
+                                                                 ChunkRule rule) {
+  __shared__ uint32_t s_key[kBoundThreads];
+  __shared__ int64_t s_bound[kBoundThreads];
+  __shared__ int64_t s_part[kBoundThreads / kWave];
+  const int64_t n = entries_present(n_cap, n_dev);
+  const int tid = threadIdx.x;
+  const int32_t t = blockIdx.x;
+  // sample i sits at n (i + 1) / (samples + 1), below n
+  auto sample_at = [&](int i) { return n * (i + 1) / (kBoundThreads + 1); };
+  uint64_t key = 0;
+  if (tid < 2 * T) {
+    const mdl_table& tb = tables[tid >> 1];
+    key = (uint64_t)tb.row_base + ((tid & 1) ? (uint64_t)tb.num_rows : 0ull);
+  }
+  s_key[tid] = n > 0 ? keys[sample_at(tid)] : 0u;
+  __syncthreads();
+  if (tid < 2 * T) {
+    int64_t lo = 0, hi = n;  // the first entry at or past the key lies in [lo, hi]
+    if (n > 0) {
+      int c0 = 0, c1 = kBoundThreads;  // samples below the key
+      while (c0 < c1) {
+        const int mid = (c0 + c1) >> 1;
+        if ((uint64_t)s_key[mid] < key) c0 = mid + 1;
+        else c1 = mid;
+      }
+      if (c0 > 0) lo = sample_at(c0 - 1) + 1;
+      if (c0 < kBoundThreads) hi = sample_at(c0);
+      // fifteen probes a round: their loads go out together, so 1500 entries
+      // between two samples take three round trips, not eleven
+      while (lo < hi) {
+        const int64_t step = (hi - lo + 15) / 16;
+        uint32_t probe[15];
+#pragma unroll
+        for (int j = 0; j < 15; ++j) {
+          const int64_t at = lo + step * (j + 1) - 1;
+          probe[j] = keys[at < hi ? at : hi - 1];
+        }
+        int below = 0;
+#pragma unroll
+        for (int j = 0; j < 15; ++j) below += lo + step * (j + 1) - 1 < hi && (uint64_t)probe[j] < key ? 1 : 0;
+        const int64_t cut = lo + step * (below + 1) - 1;
+        if (below < 15 && cut < hi) hi = cut;
+        lo += step * below;
+      }
+    }
+    s_bound[tid] = lo;
+  }
+  __syncthreads();
+  int64_t before = 0;
+  for (int32_t q = tid; q < t; q += kBoundThreads) {
+    const int64_t cq = table_chunk_len(tables[q], rule);
+    const int64_t sq = s_bound[2 * q], eq = s_bound[2 * q + 1];
+    before += ((eq > sq ? eq : sq) - sq + cq - 1) / cq;
+  }
+  for (int m = 1; m < kWave; m <<= 1) {
+    const int l = shfl_i((int)(before & 0xffffffff), lane_id() ^ m);
+    const int h = shfl_i((int)(before >> 32), lane_id() ^ m);
+    before += (int64_t)(((uint64_t)(uint32_t)h << 32) | (uint32_t)l);
+  }
+  if (lane_id() == 0) s_part[tid / kWave] = before;
+  __syncthreads();
+  int64_t base = 0;
+  for (int q = 0; q < kBoundThreads / kWave; ++q) base += s_part[q];
+  const int64_t lo = s_bound[2 * t], hi_raw = s_bound[2 * t + 1];
+  const int64_t hi = hi_raw > lo ? hi_raw : lo;
+  const int64_t cb = table_chunk_len(tables[t], rule);
+  const int64_t room = max_chunks - base;
+  const int64_t nch_all = (hi - lo + cb - 1) / cb;
+  const int64_t nch = nch_all < room ? nch_all : (room > 0 ? room : 0);
+  if (tid == 0) {
+    table_start[t] = lo;
+    table_end[t] = hi_raw;
+    chunk_base[t] = base < max_chunks ? base : max_chunks;
+    if (t == T - 1) *total = base + nch < max_chunks ? base + nch : max_chunks;
+  }
+  for (int64_t j = tid; j < nch; j += kBoundThreads) desc[base + j] = make_desc(tables[t], t, lo, hi, cb, j);
+}
+
 // Sort and chunk plan of a call of one tile in one launch: the block sorts
 // the entries, finds every table's bounds in LDS and writes the descriptors
 // that bwd_bounds_kernel and bwd_desc_kernel write for larger calls.
+template <int kItems>
 __global__ __launch_bounds__(kTileThreads) void tile_plan_kernel(TileSortArgs a, int64_t* __restrict__ table_start,
                                                                  int64_t* __restrict__ table_end,
                                                                  int64_t* __restrict__ chunk_base,
@@ -288,7 +381,7 @@ __global__ __launch_bounds__(kTileThreads) void tile_plan_kernel(TileSortArgs a,
   __shared__ int32_t s_wave[kTileWaves];
   const int64_t n = entries_present(a.n_cap, a.n_dev);
   uint32_t live = 0u, key_min = 0u;
-  if (n > 0) sort_tile(a, 0, n, st, &live, &key_min);
+  if (n > 0) sort_tile<kItems>(a, 0, n, st, &live, &key_min);
   const int tid = threadIdx.x, w = tid / kWave, lane = lane_id();
   // entries below a key
   auto below = [&](uint64_t key) {
@@ -1164,6 +1257,13 @@ static int validate_classes(const char* who, uint32_t classes) {
 
 static int plan(const mdl_table* tables, int32_t T, const uint32_t* sk, int64_t n, const int64_t* n_dev,
                 const BwdWs& w, hipStream_t s) {
+  if (2 * T <= kBoundThreads) {
+    hipLaunchKernelGGL(bwd_plan_kernel, dim3((unsigned)T), dim3(kBoundThreads), 0, s, tables, T, sk, n, n_dev,
+                       w.table_start, w.table_end, w.chunk_base, w.num_chunks, w.desc, max_chunks_for(n, T),
+                       chunk_rule(n));
+    MDL_CHECK_LAUNCH("bwd_plan_kernel");
+    return MDL_OK;
+  }
   hipLaunchKernelGGL(bwd_bounds_kernel, dim3((unsigned)(2 * T)), dim3(kBoundThreads), 0, s, tables, sk, n, n_dev,
                      w.table_start, w.table_end);
   MDL_CHECK_LAUNCH("bwd_bounds_kernel");
@@ -1221,8 +1321,12 @@ static int prepare(const mdl_table* tables, int32_t T, int32_t max_dim, uint32_t
       a.keys_out = const_cast<uint32_t*>(*sk);
       a.vals_out = const_cast<uint32_t*>(*sv);
       a.tile_min = nullptr;
-      hipLaunchKernelGGL(tile_plan_kernel, dim3(1), dim3(kTileThreads), 0, s, a, w->table_start, w->table_end,
-                         w->chunk_base, w->num_chunks, w->desc, max_chunks_for(n, T), chunk_rule(n));
+      // (a quarter or half of a tile ranks a quarter or half of its slots)
+      auto* kernel = n <= kMergeTile / 4   ? tile_plan_kernel<kTileItems / 4>
+                     : n <= kMergeTile / 2 ? tile_plan_kernel<kTileItems / 2>
+                                           : tile_plan_kernel<kTileItems>;
+      hipLaunchKernelGGL(kernel, dim3(1), dim3(kTileThreads), 0, s, a, w->table_start, w->table_end, w->chunk_base,
+                         w->num_chunks, w->desc, max_chunks_for(n, T), chunk_rule(n));
       MDL_CHECK_LAUNCH("tile_plan_kernel");
       return MDL_OK;
     }

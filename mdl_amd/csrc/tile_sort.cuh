@@ -91,27 +91,29 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
 // Sorts entries [tile * kMergeTile, +kMergeTile) of the array.  On return
 // st.key holds the tile's live keys in order, as offsets from *key_min
 // (dead ones after them), and the sorted pairs have been written out.
-// Entry i of wave w, item q, lane l is w * 256 + q * 64 + l: visited in that
-// order, so equal digits keep it (stable).
+// Entry i of wave w, item q, lane l is w * 64 * kItems + q * 64 + l: visited
+// in that order, so equal digits keep it (stable).  (kItems is a constant: with
+// a tile's own count the loops of a full tile took a fifth longer.)
+template <int kItems>
 __device__ __forceinline__ void sort_tile(const TileSortArgs& a, int64_t tile, int64_t n, TileStage& st,
                                           uint32_t* live_out, uint32_t* key_min) {
   const int tid = threadIdx.x, w = tid / kWave, lane = lane_id();
   const int64_t base = tile * kMergeTile;
   const int m = n - base < kMergeTile ? (int)(n - base) : kMergeTile;
   const uint64_t end = live_end(a.tables, a.T);
-  uint32_t k[kTileItems], v[kTileItems];
-  bool live[kTileItems];
+  uint32_t k[kItems], v[kItems];
+  bool live[kItems];
 #pragma unroll
-  for (int q = 0; q < kTileItems; ++q) {
-    const int i = w * (kWave * kTileItems) + q * kWave + lane;
+  for (int q = 0; q < kItems; ++q) {
+    const int i = w * (kWave * kItems) + q * kWave + lane;
     const int64_t at = base + (i < m ? i : m - 1);
     k[q] = a.keys_in[at];
     v[q] = a.vals_in[at];
   }
   uint32_t lo = 0xffffffffu, hi = 0u, cnt = 0u;
 #pragma unroll
-  for (int q = 0; q < kTileItems; ++q) {
-    const int i = w * (kWave * kTileItems) + q * kWave + lane;
+  for (int q = 0; q < kItems; ++q) {
+    const int i = w * (kWave * kItems) + q * kWave + lane;
     live[q] = i < m && (uint64_t)k[q] < end;
     lo = live[q] && k[q] < lo ? k[q] : lo;
     hi = live[q] && k[q] > hi ? k[q] : hi;
@@ -137,9 +139,10 @@ __device__ __forceinline__ void sort_tile(const TileSortArgs& a, int64_t tile, i
   // past the array) the offset after the largest.  Keys below 2^32 - 1
   // (the tables' rows) leave room for it.
   const uint32_t dead = tmax - tmin + 1u;
-  const uint32_t range = (int)tlive == kMergeTile ? tmax - tmin : (tlive == 0 ? 0u : dead);
+  const uint32_t range = (int)tlive == kItems * kTileThreads ? tmax - tmin : (tlive == 0 ? 0u : dead);
 #pragma unroll
-  for (int q = 0; q < kTileItems; ++q) k[q] = live[q] ? k[q] - tmin : (tlive == 0 ? 0u : dead);
+  for (int q = 0; q < kItems; ++q)
+    k[q] = live[q] ? k[q] - tmin : (tlive == 0 ? 0u : dead);
   const int bits = range == 0 ? 0 : 32 - __builtin_clz(range);
   const int passes = (bits + kTileBits - 1) / kTileBits;
   const int per = passes ? (bits + passes - 1) / passes : 0;
@@ -149,9 +152,9 @@ __device__ __forceinline__ void sort_tile(const TileSortArgs& a, int64_t tile, i
     const uint32_t mask = (1u << per) - 1u;
     for (int i = tid; i < kTileWaves * kTileRadix; i += kTileThreads) (&st.wave_hist[0][0])[i] = 0u;
     __syncthreads();
-    uint32_t rank[kTileItems];
+    uint32_t rank[kItems];
 #pragma unroll
-    for (int q = 0; q < kTileItems; ++q) {
+    for (int q = 0; q < kItems; ++q) {
       const uint32_t d = (k[q] >> shift) & mask;
       // lanes that differ from this one in any digit bit (bitop3 0xF6:
       // x | (ballot ^ t), t all ones where the lane's bit is set)
@@ -197,7 +200,7 @@ __device__ __forceinline__ void sort_tile(const TileSortArgs& a, int64_t tile, i
 #pragma unroll
     for (int g = 1; g < kDigitWaves; ++g) group_base[g] = group_base[g - 1] + st.digit_total[g - 1];
 #pragma unroll
-    for (int q = 0; q < kTileItems; ++q) {
+    for (int q = 0; q < kItems; ++q) {
       const uint32_t d = (k[q] >> shift) & mask;
       uint32_t pos = st.digit_base[d] + st.wave_hist[w][d] + rank[q];
 #pragma unroll
@@ -207,8 +210,8 @@ __device__ __forceinline__ void sort_tile(const TileSortArgs& a, int64_t tile, i
     }
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < kTileItems; ++q) {
-      const int i = w * (kWave * kTileItems) + q * kWave + lane;
+    for (int q = 0; q < kItems; ++q) {
+      const int i = w * (kWave * kItems) + q * kWave + lane;
       k[q] = st.key[i];
       v[q] = st.val[i];
     }
@@ -216,12 +219,13 @@ __device__ __forceinline__ void sort_tile(const TileSortArgs& a, int64_t tile, i
   if (passes == 0) {
     // one key value (or none live): the input order stands
 #pragma unroll
-    for (int q = 0; q < kTileItems; ++q) st.key[w * (kWave * kTileItems) + q * kWave + lane] = k[q];
+    for (int q = 0; q < kItems; ++q)
+      st.key[w * (kWave * kItems) + q * kWave + lane] = k[q];
     __syncthreads();
   }
 #pragma unroll
-  for (int q = 0; q < kTileItems; ++q) {
-    const int i = w * (kWave * kTileItems) + q * kWave + lane;
+  for (int q = 0; q < kItems; ++q) {
+    const int i = w * (kWave * kItems) + q * kWave + lane;
     if (i < m) {
       a.keys_out[base + i] = i < (int)tlive ? k[q] + tmin : (uint32_t)end;
       a.vals_out[base + i] = v[q];
@@ -241,7 +245,7 @@ static __global__ __launch_bounds__(kTileThreads) void tile_sort_kernel(TileSort
   const int64_t n = entries_present(a.n_cap, a.n_dev);
   if ((int64_t)blockIdx.x * kMergeTile >= n) return;
   uint32_t live, key_min;
-  sort_tile(a, blockIdx.x, n, st, &live, &key_min);
+  sort_tile<kTileItems>(a, blockIdx.x, n, st, &live, &key_min);
 }
 
 // Entries of sorted s[lo, hi) that go before x: those below it, and with
