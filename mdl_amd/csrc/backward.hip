@@ -90,10 +90,15 @@ struct BwdWs {
 // 40.8 (its norm pass 49.3 / 29.5 / 21.6 / 23.9); 262 K of one bf16 table
 // 27.1 / 19.5 / 16.5 / 16.4 (27.4 with slices of 16 at least); 131 K uniform
 // ids 22.2 / 19.7 / 19.6 / 19.7 (29.2).  Shorter slices leave more runs
-// crossing slots and chunks.
+// crossing slots and chunks; only the smallest calls, whose chunks leave most
+// CUs without a wave, gain from two entries (3 K entries 11.7 -> 9.3 us; 131 K
+// 19.5 -> 21.4).
 constexpr int kSlotRunMin = 4;
+constexpr int kSlotRunTiny = 2;
+constexpr int64_t kTinyEntries = 16384;
 constexpr int64_t kSlotTarget = 65536;
 static inline int slot_run_for(int64_t n) {
+  if (n <= kTinyEntries) return kSlotRunTiny;
   const int64_t r = n / kSlotTarget;
   return (int)(r < kSlotRunMin ? kSlotRunMin : (r > kSlotRun ? kSlotRun : r));
 }
@@ -1321,10 +1326,11 @@ static int prepare(const mdl_table* tables, int32_t T, int32_t max_dim, uint32_t
       a.keys_out = const_cast<uint32_t*>(*sk);
       a.vals_out = const_cast<uint32_t*>(*sv);
       a.tile_min = nullptr;
-      // (a quarter or half of a tile ranks a quarter or half of its slots)
-      auto* kernel = n <= kMergeTile / 4   ? tile_plan_kernel<kTileItems / 4>
-                     : n <= kMergeTile / 2 ? tile_plan_kernel<kTileItems / 2>
-                                           : tile_plan_kernel<kTileItems>;
+      // (a shorter tile ranks fewer slots)
+      auto* kernel = n <= kMergeTile / 4       ? tile_plan_kernel<kTileItems / 4>
+                     : n <= kMergeTile / 2     ? tile_plan_kernel<kTileItems / 2>
+                     : n <= kMergeTile / 4 * 3 ? tile_plan_kernel<kTileItems / 4 * 3>
+                                               : tile_plan_kernel<kTileItems>;
       hipLaunchKernelGGL(kernel, dim3(1), dim3(kTileThreads), 0, s, a, w->table_start, w->table_end, w->chunk_base,
                          w->num_chunks, w->desc, max_chunks_for(n, T), chunk_rule(n));
       MDL_CHECK_LAUNCH("tile_plan_kernel");

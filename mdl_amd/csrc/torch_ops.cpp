@@ -385,8 +385,9 @@ void check_features(TensorList weights, TensorList ids, const c10::List<std::opt
   }
 }
 
+// (mdl_amd.ops.forward_target_ids: the same rule, with its figures)
 int forward_target_ids(int64_t n) {
-  return (int)std::max<int64_t>(96, std::min<int64_t>(kForwardTargetIds, n / 3072));
+  return (int)std::max<int64_t>(32, std::min<int64_t>(kForwardTargetIds, n / 3072));
 }
 
 // Per-call descriptor columns (build_features): output/gradient rows, id and

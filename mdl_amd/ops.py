@@ -43,12 +43,14 @@ FORWARD_TARGET_IDS = 480
 
 def forward_target_ids(feats: np.ndarray) -> int:
     """Ids per forward chunk for this call: FORWARD_TARGET_IDS, or fewer (down
-    to 96) when a small call would give fewer than ~3000 chunks -- a wave per
-    chunk, and every CU needs several (c0, 0.4 M ids: 480 ids per chunk took
-    the lookup 0.045 ms, 120 took 0.031 ms)."""
+    to 32) when a small call would give fewer than ~3000 chunks -- a wave per
+    chunk, and every CU needs several (0.4 M ids of 32 tables: 480 ids per
+    chunk took the lookup 0.045 ms, 120 took 0.031 ms; 3 K ids: 96 took
+    12.1 us, 48 9.7, 32 9.2; half as many ids per chunk at 0.4-0.9 M ids took
+    5-10 % longer)."""
 
     n = int(np.asarray(feats["num_ids"], dtype=np.int64).sum()) if len(feats) else 0
-    return max(96, min(FORWARD_TARGET_IDS, n // 3072))
+    return max(32, min(FORWARD_TARGET_IDS, n // 3072))
 
 
 def _require_device(t: Tensor, what: str) -> None:
