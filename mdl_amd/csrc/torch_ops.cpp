@@ -1648,12 +1648,15 @@ std::tuple<Tensor, Tensor> bucketize_cuda(const Tensor& raw_in, const std::optio
   return {out, err};
 }
 
-std::tuple<Tensor, Tensor, Tensor, Tensor> bag_truncate_cuda(const Tensor& values_in, const Tensor& offsets_in,
+// (ids, lengths, kept offsets, error count): the offsets and the error count
+// in one int64 buffer, the count (int32) after the last offset, when `joined`
+// -- a caller that reads both copies their two words at once.
+std::tuple<Tensor, Tensor, Tensor, Tensor> truncate_bags(const Tensor& values_in, const Tensor& offsets_in,
                                                              const std::optional<Tensor>& valid_in,
                                                              const std::optional<Tensor>& row_valid_in,
                                                              int64_t max_length, c10::string_view truncation,
                                                              c10::string_view bucket, int64_t num_buckets,
-                                                             bool validate_nonzero) {
+                                                             bool validate_nonzero, bool joined) {
   require_device(values_in, "list values");
   TORCH_CHECK_TYPE(values_in.scalar_type() == at::kLong && offsets_in.scalar_type() == at::kLong,
                    "list values and offsets must be torch.int64");
@@ -1675,8 +1678,14 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> bag_truncate_cuda(const Tensor& value
   if (row_valid_in.has_value() && row_valid_in->defined()) row_valid = row_valid_in->to(dev, at::kByte).contiguous();
   const int64_t n_in = values.numel();
   auto i64 = at::TensorOptions().dtype(at::kLong).device(dev);
-  Tensor ids = at::empty({n_in}, i64), lengths = at::empty({rows}, i64), out_offsets = at::empty({rows + 1}, i64);
-  Tensor err = at::zeros({1}, at::TensorOptions().dtype(at::kInt).device(dev));
+  Tensor ids = at::empty({n_in}, i64), lengths = at::empty({rows}, i64);
+  Tensor out_offsets = at::empty({rows + 1 + (joined ? 1 : 0)}, i64), err;
+  if (joined) {
+    out_offsets.narrow(0, rows + 1, 1).zero_();
+    err = raw_view(out_offsets, at::kInt, 8 * (rows + 1), {1}, {1});
+  } else {
+    err = at::zeros({1}, at::TensorOptions().dtype(at::kInt).device(dev));
+  }
   Tensor ws = workspace(mdl_bag_truncate_workspace_bytes(rows), dev);
   check(mdl_bag_truncate(offsets.data_ptr<int64_t>(), row_valid.defined() ? row_valid.data_ptr<uint8_t>() : nullptr,
                          rows, n_in ? values.data_ptr<int64_t>() : nullptr,
@@ -1687,6 +1696,31 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> bag_truncate_cuda(const Tensor& value
                          err.data_ptr<int32_t>(), ws.data_ptr(), (size_t)ws.numel(), stream_of(dev)),
         "mdl_bag_truncate");
   return {ids, lengths, out_offsets, err};
+}
+
+std::tuple<Tensor, Tensor, Tensor, Tensor> bag_truncate_cuda(const Tensor& values, const Tensor& offsets,
+                                                             const std::optional<Tensor>& valid,
+                                                             const std::optional<Tensor>& row_valid,
+                                                             int64_t max_length, c10::string_view truncation,
+                                                             c10::string_view bucket, int64_t num_buckets,
+                                                             bool validate_nonzero) {
+  return truncate_bags(values, offsets, valid, row_valid, max_length, truncation, bucket, num_buckets,
+                       validate_nonzero, false);
+}
+
+// bag_truncate for a caller that sizes the ids on the host: (ids cut to the
+// kept total, lengths, errors), with one read of both numbers.
+std::tuple<Tensor, Tensor, int64_t> bag_truncate_exact(const Tensor& values, const Tensor& offsets,
+                                                       const std::optional<Tensor>& valid,
+                                                       const std::optional<Tensor>& row_valid, int64_t max_length,
+                                                       c10::string_view truncation, c10::string_view bucket,
+                                                       int64_t num_buckets, bool validate_nonzero) {
+  auto [ids, lengths, out_offsets, err] = truncate_bags(values, offsets, valid, row_valid, max_length, truncation,
+                                                        bucket, num_buckets, validate_nonzero, true);
+  const Tensor h = out_offsets.narrow(0, lengths.numel(), 2).to(at::kCPU);
+  const int64_t* w = h.data_ptr<int64_t>();
+  // (malformed offsets can add up to more than the values hold)
+  return {ids.narrow(0, 0, std::min<int64_t>(w[0], ids.numel())), lengths, w[1]};
 }
 
 Tensor lengths_to_offsets_cuda(const Tensor& lengths_in) {
@@ -2133,6 +2167,9 @@ TORCH_LIBRARY(mdl_hip, m) {
         "Tensor payload, int num_entries, Tensor? bag_count, Tensor(a!) sumsq, int slot, Tensor(b!) workspace, "
         "int max_dim, int key_bits, int classes) -> ()",
         &backward_sumsq_);
+  m.def("bag_truncate_exact(Tensor values, Tensor offsets, Tensor? valid, Tensor? row_valid, int max_length, "
+        "str truncation, str bucket, int num_buckets, bool validate_nonzero) -> (Tensor, Tensor, int)",
+        &bag_truncate_exact);
   // Pooling of already-embedded rows (mdl_amd/pooling.py's autograd function).
   m.def("pool_bags_forward(Tensor[] embedded, Tensor[] ids, Tensor[] lengths, int[] codes, bool mean, "
         "Tensor(a!)? counter) -> (Tensor[], Tensor, Tensor, Tensor)",

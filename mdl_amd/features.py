@@ -142,12 +142,17 @@ def bag_csr_tensor(
         raise ValueError(f"max_length must be non-negative, got {max_length}")
     if bucket == "pre_hashed" and (num_buckets <= 0 or num_buckets & (num_buckets - 1)):
         raise ValueError("pre_hashed num_buckets must be a positive power of two")
-    ids, lengths, out_offsets, err = torch.ops.mdl_hip.bag_truncate(
-        values, offsets, valid, row_valid, -1 if max_length is None else int(max_length), truncation, bucket,
-        int(num_buckets), bool(validate_nonzero))
-    if not exact:
-        return {"values": ids, "lengths": lengths, "offsets": out_offsets, "errors": err}
-    total, bad = (int(x) for x in torch.stack([out_offsets[-1], err[0].to(torch.int64)]).cpu())
+    args = (values, offsets, valid, row_valid, -1 if max_length is None else int(max_length), truncation, bucket,
+            int(num_buckets), bool(validate_nonzero))
+    if exact and values.is_cuda and type(values) is Tensor and not torch.compiler.is_compiling():
+        # one call, its two numbers read back together
+        ids, lengths, bad = torch.ops.mdl_hip.bag_truncate_exact(*args)
+        total = ids.numel()
+    else:
+        ids, lengths, out_offsets, err = torch.ops.mdl_hip.bag_truncate(*args)
+        if not exact:
+            return {"values": ids, "lengths": lengths, "offsets": out_offsets, "errors": err}
+        total, bad = (int(x) for x in torch.stack([out_offsets[-1], err[0].to(torch.int64)]).cpu())
     if bad:
         n = values.numel()
         malformed = bool(((offsets < 0) | (offsets > n)).any()) or bool((offsets[1:] < offsets[:-1]).any())
