@@ -483,6 +483,17 @@ int mdl_backward_sumsq(const mdl_feature* feats, int32_t num_features,
                        void* stream);
 
 /*
+ * mdl_backward_sumsq into sumsq[count - 1], then mdl_clip_coef of all count
+ * squared norms, in the same launches: the last key group of a clipped step.
+ */
+int mdl_backward_sumsq_coef(const mdl_feature* feats, int32_t num_features,
+                            const mdl_table* tables, int32_t num_tables, int32_t max_dim,
+                            uint32_t* sort_keys, uint32_t* sort_payload, int64_t n,
+                            int32_t key_bits, const float* bag_count, float* sumsq, int32_t count,
+                            float max_norm, float* total_norm, float* coef, void* workspace,
+                            size_t workspace_bytes, uint32_t classes, void* stream);
+
+/*
  * Coalesced sparse gradients, the autograd contract of src/optim.py:317-329 and
  * src/train.py:5730-5742 (rows ascending and unique), in two calls:
  * mdl_backward_count sorts and writes unique_range[2t], unique_range[2t+1]
@@ -579,6 +590,11 @@ int mdl_sumsq(const mdl_span* spans, int32_t num_spans, float* sumsq,
 int mdl_clip_coef(const float* sumsq, int32_t count, float max_norm,
                   float* total_norm, float* coef, void* stream);
 int mdl_scale(const mdl_span* spans, int32_t num_spans, const float* coef, void* stream);
+/* mdl_sumsq into sumsq[count - 1], then mdl_clip_coef of all count squared
+ * norms, in the same launches (the last list of a clip). */
+int mdl_sumsq_coef(const mdl_span* spans, int32_t num_spans, float* sumsq, int32_t count,
+                   float max_norm, float* total_norm, float* coef, void* workspace,
+                   size_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------- update --- */
 

@@ -151,7 +151,12 @@ SIGNATURES: dict[str, tuple] = {
         _I32,
         [_P, _I32, _P, _I32, _I32, _P, _P, _I64, _I32, _P, _P, _P, _SZ, _U32, _P],
     ),
+    "mdl_backward_sumsq_coef": (
+        _I32,
+        [_P, _I32, _P, _I32, _I32, _P, _P, _I64, _I32, _P, _P, _I32, _F, _P, _P, _P, _SZ, _U32, _P],
+    ),
     "mdl_sumsq_workspace_bytes": (_SZ, [_I32]),
+    "mdl_sumsq_coef": (_I32, [_P, _I32, _P, _I32, _F, _P, _P, _P, _SZ, _P]),
     "mdl_sumsq": (_I32, [_P, _I32, _P, _P, _SZ, _P]),
     "mdl_clip_coef": (_I32, [_P, _I32, _F, _P, _P, _P]),
     "mdl_scale": (_I32, [_P, _I32, _P, _P]),

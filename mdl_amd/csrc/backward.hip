@@ -32,7 +32,8 @@ int sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* val
                const int64_t* n_dev, int key_bits, void* ws, size_t ws_bytes, int* in_alt, hipStream_t s);
 size_t sort_ws_bytes(int64_t n);
 int sort_pass_count(int key_bits);
-int launch_sum_partials(const float* partial, int64_t m, const int64_t* m_dev, float* out, hipStream_t s);
+int launch_sum_partials(const float* partial, int64_t m, const int64_t* m_dev, float* out, const ClipTail& c,
+                        hipStream_t s);
 
 constexpr int kChunkMax = 512;    // entries of one chunk at most
 constexpr int kSlotRun = kPassesPerChunk;  // entries one slot walks in a full chunk
@@ -1619,16 +1620,16 @@ int mdl_backward_apply(const mdl_feature* feats, int32_t num_features, const mdl
   return run_reduce(a, classes, as_stream(stream));
 }
 
-int mdl_backward_sumsq(const mdl_feature* feats, int32_t num_features, const mdl_table* tables,
-                       int32_t num_tables, int32_t max_dim, uint32_t* sort_keys, uint32_t* sort_payload,
-                       int64_t n, int32_t key_bits, const float* bag_count, float* sumsq, void* workspace,
-                       size_t workspace_bytes, uint32_t classes, void* stream) {
+static int backward_sumsq(const mdl_feature* feats, int32_t num_features, const mdl_table* tables,
+                          int32_t num_tables, int32_t max_dim, uint32_t* sort_keys, uint32_t* sort_payload, int64_t n,
+                          int32_t key_bits, const float* bag_count, float* sumsq, const ClipTail& tail,
+                          void* workspace, size_t workspace_bytes, uint32_t classes, void* stream) {
   int rc = validate_tables("mdl_backward_sumsq", num_tables, max_dim, n);
   if (!rc) rc = validate_classes("mdl_backward_sumsq", classes);
   if (rc) return rc;
   if (!sumsq) return fail(MDL_ERR_INVALID, "mdl_backward_sumsq: null output");
   hipStream_t s = as_stream(stream);
-  if (n == 0) return launch_sum_partials(nullptr, 0, nullptr, sumsq, s);
+  if (n == 0) return launch_sum_partials(nullptr, 0, nullptr, sumsq, tail, s);
   BwdArgs a;
   rc = sorted_args("mdl_backward_sumsq", &a, feats, num_features, tables, num_tables, max_dim, sort_keys,
                    sort_payload, n, key_bits, bag_count, workspace, workspace_bytes);
@@ -1637,7 +1638,26 @@ int mdl_backward_sumsq(const mdl_feature* feats, int32_t num_features, const mdl
   rc = run_reduce(a, classes, s);
   if (rc) return rc;
   // *num_chunks chunks were reduced; their partials are added in chunk order.
-  return launch_sum_partials(a.chunk_ss, 0, a.num_chunks, sumsq, s);
+  return launch_sum_partials(a.chunk_ss, 0, a.num_chunks, sumsq, tail, s);
+}
+
+int mdl_backward_sumsq(const mdl_feature* feats, int32_t num_features, const mdl_table* tables,
+                       int32_t num_tables, int32_t max_dim, uint32_t* sort_keys, uint32_t* sort_payload,
+                       int64_t n, int32_t key_bits, const float* bag_count, float* sumsq, void* workspace,
+                       size_t workspace_bytes, uint32_t classes, void* stream) {
+  return backward_sumsq(feats, num_features, tables, num_tables, max_dim, sort_keys, sort_payload, n, key_bits,
+                        bag_count, sumsq, ClipTail{}, workspace, workspace_bytes, classes, stream);
+}
+
+int mdl_backward_sumsq_coef(const mdl_feature* feats, int32_t num_features, const mdl_table* tables,
+                            int32_t num_tables, int32_t max_dim, uint32_t* sort_keys, uint32_t* sort_payload,
+                            int64_t n, int32_t key_bits, const float* bag_count, float* sumsq, int32_t count,
+                            float max_norm, float* total_norm, float* coef, void* workspace, size_t workspace_bytes,
+                            uint32_t classes, void* stream) {
+  if (count < 1 || !sumsq || !coef) return fail(MDL_ERR_INVALID, "mdl_backward_sumsq_coef: bad arguments");
+  return backward_sumsq(feats, num_features, tables, num_tables, max_dim, sort_keys, sort_payload, n, key_bits,
+                        bag_count, sumsq + (count - 1), ClipTail{sumsq, count, max_norm, total_norm, coef}, workspace,
+                        workspace_bytes, classes, stream);
 }
 
 int mdl_backward_adagrad(const mdl_feature* feats, int32_t num_features, const mdl_table* tables,

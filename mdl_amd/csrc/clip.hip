@@ -92,8 +92,21 @@ __global__ __launch_bounds__(kNormThreads) void span_sumsq_kernel(const mdl_span
 // threads: the per-chunk partials of a c1 backward (17-42 K of them) take
 // about five memory round trips instead of twenty (22.6 us with 256 threads).
 constexpr int kSumThreads = 1024;
+
+// total = sqrt(sum of the count squared norms), added in fp32 in order like
+// the trainer's replicated + sharded sum; coef = min(max_norm / (total + 1e-6), 1).
+__device__ __forceinline__ void clip_coefficient(float t, const ClipTail& c) {
+  const float norm = sqrtf(t);
+  const float k = c.max_norm / (norm + 1e-6f);
+  if (c.total_norm) c.total_norm[0] = norm;
+  c.coef[0] = k < 1.f ? k : 1.f;
+}
+
+// With c.coef the sum just made is the last of c.count squared norms at
+// c.sumsq, and the clip coefficient follows from them here: a launch of its
+// own took 3-5 us of a clipped step.
 __global__ __launch_bounds__(kSumThreads) void sum_partials_kernel(const float* __restrict__ partial, int64_t m,
-                                                                    const int64_t* m_dev, float* out) {
+                                                                    const int64_t* m_dev, float* out, ClipTail c) {
   __shared__ double smem[kSumThreads];
   if (m_dev) m = *m_dev;
   constexpr int kBatch = 8;
@@ -114,20 +127,22 @@ __global__ __launch_bounds__(kSumThreads) void sum_partials_kernel(const float* 
     if (threadIdx.x < d) smem[threadIdx.x] += smem[threadIdx.x + d];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[0] = (float)smem[0];
+  if (threadIdx.x == 0) {
+    const float last = (float)smem[0];
+    out[0] = last;
+    if (c.coef != nullptr) {
+      float t = 0.f;
+      for (int32_t i = 0; i + 1 < c.count; ++i) t += c.sumsq[i];
+      clip_coefficient(t + last, c);
+    }
+  }
 }
 
-// total = sqrt(sum of the count squared norms), added in fp32 in order like
-// the trainer's replicated + sharded sum; coef = min(max_norm / (total + 1e-6), 1).
-__global__ void clip_coef_kernel(const float* __restrict__ sumsq, int32_t count, float max_norm, float* total_norm,
-                                 float* coef) {
+__global__ void clip_coef_kernel(ClipTail c) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   float t = 0.f;
-  for (int32_t i = 0; i < count; ++i) t += sumsq[i];
-  const float norm = sqrtf(t);
-  const float c = max_norm / (norm + 1e-6f);
-  if (total_norm) total_norm[0] = norm;
-  coef[0] = c < 1.f ? c : 1.f;
+  for (int32_t i = 0; i < c.count; ++i) t += c.sumsq[i];
+  clip_coefficient(t, c);
 }
 
 // x *= coef in the span's dtype: for bf16 the coefficient is rounded to bf16
@@ -173,8 +188,9 @@ __global__ __launch_bounds__(kNormThreads) void span_scale_kernel(const mdl_span
   }
 }
 
-int launch_sum_partials(const float* partial, int64_t m, const int64_t* m_dev, float* out, hipStream_t s) {
-  hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(kSumThreads), 0, s, partial, m, m_dev, out);
+int launch_sum_partials(const float* partial, int64_t m, const int64_t* m_dev, float* out, const ClipTail& c,
+                        hipStream_t s) {
+  hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(kSumThreads), 0, s, partial, m, m_dev, out, c);
   MDL_CHECK_LAUNCH("sum_partials_kernel");
   return MDL_OK;
 }
@@ -189,10 +205,10 @@ size_t mdl_sumsq_workspace_bytes(int32_t num_spans) {
   return (size_t)(num_spans > 0 ? num_spans : 1) * kNormParts * sizeof(float) + 256;
 }
 
-int mdl_sumsq(const mdl_span* spans, int32_t num_spans, float* sumsq, void* workspace, size_t workspace_bytes,
-              void* stream) {
+static int sumsq(const mdl_span* spans, int32_t num_spans, float* out, const ClipTail& c, void* workspace,
+                 size_t workspace_bytes, void* stream) {
   if (num_spans < 0 || num_spans > 65535) return fail(MDL_ERR_INVALID, "mdl_sumsq: num_spans outside [0, 65535]");
-  if (!sumsq) return fail(MDL_ERR_INVALID, "mdl_sumsq: null output");
+  if (!out) return fail(MDL_ERR_INVALID, "mdl_sumsq: null output");
   if (workspace_bytes < mdl_sumsq_workspace_bytes(num_spans))
     return fail(MDL_ERR_WORKSPACE, "mdl_sumsq: workspace too small");
   hipStream_t s = as_stream(stream);
@@ -203,13 +219,25 @@ int mdl_sumsq(const mdl_span* spans, int32_t num_spans, float* sumsq, void* work
                        partial);
     MDL_CHECK_LAUNCH("span_sumsq_kernel");
   }
-  return launch_sum_partials(partial, (int64_t)num_spans * kNormParts, nullptr, sumsq, s);
+  return launch_sum_partials(partial, (int64_t)num_spans * kNormParts, nullptr, out, c, s);
+}
+
+int mdl_sumsq(const mdl_span* spans, int32_t num_spans, float* sumsq_out, void* workspace, size_t workspace_bytes,
+              void* stream) {
+  return sumsq(spans, num_spans, sumsq_out, ClipTail{}, workspace, workspace_bytes, stream);
+}
+
+int mdl_sumsq_coef(const mdl_span* spans, int32_t num_spans, float* sumsq_out, int32_t count, float max_norm,
+                   float* total_norm, float* coef, void* workspace, size_t workspace_bytes, void* stream) {
+  if (count < 1 || !sumsq_out || !coef) return fail(MDL_ERR_INVALID, "mdl_sumsq_coef: bad arguments");
+  return sumsq(spans, num_spans, sumsq_out + (count - 1), ClipTail{sumsq_out, count, max_norm, total_norm, coef},
+               workspace, workspace_bytes, stream);
 }
 
 int mdl_clip_coef(const float* sumsq, int32_t count, float max_norm, float* total_norm, float* coef, void* stream) {
   if (count < 0 || (count > 0 && !sumsq) || !coef) return fail(MDL_ERR_INVALID, "mdl_clip_coef: bad arguments");
-  hipLaunchKernelGGL(clip_coef_kernel, dim3(1), dim3(kWave), 0, as_stream(stream), sumsq, count, max_norm,
-                     total_norm, coef);
+  hipLaunchKernelGGL(clip_coef_kernel, dim3(1), dim3(kWave), 0, as_stream(stream),
+                     ClipTail{sumsq, count, max_norm, total_norm, coef});
   MDL_CHECK_LAUNCH("clip_coef_kernel");
   return MDL_OK;
 }

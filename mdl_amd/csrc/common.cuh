@@ -25,6 +25,16 @@ int check_hip(hipError_t err, const char* what);
     if (_e != hipSuccess) return ::mdl::check_hip(_e, what);     \
   } while (0)
 
+// The clip coefficient that ends a sum of squares: the last of count squared
+// norms at sumsq (coef NULL: none follows).
+struct ClipTail {
+  const float* sumsq = nullptr;
+  int32_t count = 0;
+  float max_norm = 0.f;
+  float* total_norm = nullptr;
+  float* coef = nullptr;
+};
+
 static inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
 // ------------------------------------------------------------- numerics --

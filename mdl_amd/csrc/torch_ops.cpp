@@ -1611,18 +1611,16 @@ Tensor clip_sparse_grad_norm_(TensorList replicated, TensorList sharded, double 
   Tensor sumsq = at::empty({2}, f32), norm = at::empty({1}, f32), coef = at::empty({1}, f32);
   const size_t wsb = mdl_sumsq_workspace_bytes((int32_t)std::max(rs.size(), ss.size()));
   Tensor ws = workspace(wsb, dev);
-  // a list without gradients adds nothing to the norm and launches nothing
-  // (both empty: one sum of no spans)
-  int32_t lists = 0;
-  auto sum_list = [&](const std::vector<mdl_span>& spans, const mdl_span* at) {
-    check(mdl_sumsq(spans.empty() ? nullptr : at, (int32_t)spans.size(), sumsq.data_ptr<float>() + lists++,
-                    ws.data_ptr(), wsb, s),
-          "mdl_sumsq");
-  };
-  if (!rs.empty()) sum_list(rs, sd);
-  if (!ss.empty() || rs.empty()) sum_list(ss, sd + rs.size());
-  check(mdl_clip_coef(sumsq.data_ptr<float>(), lists, (float)max_norm, norm.data_ptr<float>(), coef.data_ptr<float>(), s),
-        "mdl_clip_coef");
+  // A list without gradients adds nothing to the norm and launches nothing
+  // (both empty: one sum of no spans); the last list's sum ends in the
+  // coefficient.
+  const bool two = !rs.empty() && !ss.empty();
+  const auto& last = ss.empty() ? rs : ss;
+  if (two) check(mdl_sumsq(sd, (int32_t)rs.size(), sumsq.data_ptr<float>(), ws.data_ptr(), wsb, s), "mdl_sumsq");
+  check(mdl_sumsq_coef(last.empty() ? nullptr : (two ? sd + rs.size() : sd), (int32_t)last.size(),
+                       sumsq.data_ptr<float>(), two ? 2 : 1, (float)max_norm, norm.data_ptr<float>(),
+                       coef.data_ptr<float>(), ws.data_ptr(), wsb, s),
+        "mdl_sumsq_coef");
   if (!all.empty()) check(mdl_scale(sd, (int32_t)all.size(), coef.data_ptr<float>(), s), "mdl_scale");
   return norm.reshape({});
 }
@@ -2070,16 +2068,32 @@ void fused_backward_rowwise_adagrad_(TensorList weights, TensorList accumulators
                   bag_count, grad_scale, ws, max_dim, key_bits, classes, lr, eps);
 }
 
+// The squared norm of slot `slot`; with `coef` also the clip coefficient of
+// the slots up to and with it.
 void backward_sumsq_(const Tensor& features, int64_t num_features, const Tensor& tables, int64_t num_tables,
                      const Tensor& keys, const Tensor& payload, int64_t num_entries,
                      const std::optional<Tensor>& bag_count, const Tensor& sumsq, int64_t slot, const Tensor& ws,
-                     int64_t max_dim, int64_t key_bits, int64_t classes) {
+                     int64_t max_dim, int64_t key_bits, int64_t classes, double max_norm,
+                     const std::optional<Tensor>& total_norm, const std::optional<Tensor>& coef) {
   const at::Device dev = keys.device();
   const c10::DeviceGuard guard(dev);
-  check(mdl_backward_sumsq(reinterpret_cast<const mdl_feature*>(features.data_ptr()), (int32_t)num_features,
-                           reinterpret_cast<const mdl_table*>(tables.data_ptr()), (int32_t)num_tables, (int32_t)max_dim,
-                           reinterpret_cast<uint32_t*>(keys.data_ptr()), reinterpret_cast<uint32_t*>(payload.data_ptr()),
-                           num_entries, (int32_t)key_bits, ptr_or_null<float>(bag_count), at_offset<float>(sumsq, slot),
+  const auto* fd = reinterpret_cast<const mdl_feature*>(features.data_ptr());
+  const auto* td = reinterpret_cast<const mdl_table*>(tables.data_ptr());
+  auto* kp = reinterpret_cast<uint32_t*>(keys.data_ptr());
+  auto* pp = reinterpret_cast<uint32_t*>(payload.data_ptr());
+  if (coef.has_value() && coef->defined()) {
+    TORCH_CHECK_VALUE(sumsq.scalar_type() == at::kFloat && sumsq.is_contiguous() && sumsq.numel() > slot,
+                      "squared norms are a contiguous float32 tensor");
+    check(mdl_backward_sumsq_coef(fd, (int32_t)num_features, td, (int32_t)num_tables, (int32_t)max_dim, kp, pp,
+                                  num_entries, (int32_t)key_bits, ptr_or_null<float>(bag_count),
+                                  sumsq.data_ptr<float>(), (int32_t)slot + 1, (float)max_norm,
+                                  ptr_or_null<float>(total_norm), coef->data_ptr<float>(), ws.data_ptr(),
+                                  (size_t)ws.numel(), (uint32_t)classes, stream_of(dev)),
+          "mdl_backward_sumsq_coef");
+    return;
+  }
+  check(mdl_backward_sumsq(fd, (int32_t)num_features, td, (int32_t)num_tables, (int32_t)max_dim, kp, pp, num_entries,
+                           (int32_t)key_bits, ptr_or_null<float>(bag_count), at_offset<float>(sumsq, slot),
                            ws.data_ptr(), (size_t)ws.numel(), (uint32_t)classes, stream_of(dev)),
         "mdl_backward_sumsq");
 }
@@ -2165,7 +2179,8 @@ TORCH_LIBRARY(mdl_hip, m) {
         &fused_backward_rowwise_adagrad_);
   m.def("backward_sumsq_(Tensor features, int num_features, Tensor tables, int num_tables, Tensor keys, "
         "Tensor payload, int num_entries, Tensor? bag_count, Tensor(a!) sumsq, int slot, Tensor(b!) workspace, "
-        "int max_dim, int key_bits, int classes) -> ()",
+        "int max_dim, int key_bits, int classes, float max_norm=0., Tensor(c!)? total_norm=None, "
+        "Tensor(d!)? coef=None) -> ()",
         &backward_sumsq_);
   m.def("bag_truncate_exact(Tensor values, Tensor offsets, Tensor? valid, Tensor? row_valid, int max_length, "
         "str truncation, str bucket, int num_buckets, bool validate_nonzero) -> (Tensor, Tensor, int)",

@@ -371,8 +371,9 @@ class SparseStep:
             torch.ops.mdl_hip.backward_sumsq_(
                 gs.feats_bwd_dev, len(gs.feats_bwd), gs.tables_dev, len(gs.tables), gs.keys, gs.payload, self._n(),
                 self.bag_count, self.sumsq, g, gs.ws, self.plan.max_dim, self.plan.key_bits, gs.bwd_classes,
+                # the last group's sum ends in the coefficient
+                *((float(max_norm), self.norm, self.coef) if g == len(self.groups) - 1 else ()),
             )
-        torch.ops.mdl_hip.clip_coefficient_(self.sumsq, len(self.groups), float(max_norm), self.norm, self.coef)
         return self.norm, self.coef
 
     def step(self, lr: float, eps: float, clip_norm: float | None = None) -> None:
