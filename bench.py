@@ -892,9 +892,10 @@ def cpu_baseline(wl: Workload, batch, steps: int = 5, warmup: int = 2, row_cap: 
 # The bench line then reports that file's figure as roofline.traffic.
 
 KERNEL_GROUPS = {
-    "forward": ("forward_kernel", "sequence_kernel", "sequence_keys_kernel"),
+    "forward": ("forward_kernel", "sequence_kernel"),
     "apply": ("bwd_reduce_kernel<false", "bwd_reduce_kernel<true"),
-    "sort": ("radix_upsweep", "radix_scan", "radix_downsweep"),
+    "sort": ("radix_upsweep", "radix_scan", "radix_downsweep", "tile_sort_kernel", "rank_merge_kernel",
+             "tile_plan_kernel"),
 }
 COPY_BYTES = 1 << 30
 
@@ -1115,7 +1116,7 @@ def measure(name: str, args, torch, device, *, with_aux: bool = False) -> dict:
                                    + wl.batch * a["sum_dim"] * esz + 4 * nb for a in used]))
         apply_bytes = float(np.mean([8 * a["n_ids"] + wl.batch * a["sum_dim"] * esz
                                      + 2 * a["fwd_unique_row_bytes"] + 8 * a["unique_rows"] + 4 * nb for a in used]))
-    fwd_label = ("sequence_kernel + sequence_keys_kernel per feature (window gather, mask, sort keys)"
+    fwd_label = ("sequence_kernel per feature (window gather, mask, sort keys)"
                  if wl.kind == "sequence" else "forward_kernel (grouped lookup + pooling + sort-key emission)")
     for kname, nbytes, label in (
         ("forward", fwd_bytes, fwd_label),

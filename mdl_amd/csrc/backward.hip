@@ -2,16 +2,16 @@
 // reduction of per-id gradients, fused with the row-wise Adagrad update (or
 // writing a coalesced sparse gradient, or only its squared norm).
 //
-// After the stable radix sort every distinct (table, row) is one run of equal
+// After the stable sort every distinct (table, row) is one run of equal
 // keys whose payloads (gradient rows) appear in input order.  The sorted
 // array is cut into chunks of <= kChunkMax entries that never straddle two
 // tables, numbered so that the chunks of one kernel variant (row-access
 // class x lane width) are contiguous and each table's chunks consecutive.
 //
 // One wavefront reduces one chunk.  Its G = 64/L lane groups ("slots", L
-// lanes per row) each walk a contiguous slice of about kSlotRun (48) entries (fewer in a small call),
-// accumulating the per-id gradients in registers: the gradient rows of the
-// slice are the only per-entry work, and a run that ends inside the slot that
+// lanes per row) each walk a contiguous slice of up to kSlotRun (48) entries
+// (fewer in a small call, see slot_run_for), accumulating the per-id gradients
+// in registers: the gradient rows of the slice are the only per-entry work, and a run that ends inside the slot that
 // began it is finished right there -- its summed gradient goes straight into
 // the Adagrad update, with the weight row and accumulator loaded alongside
 // the gradient rows (read and written once).  Runs that cross slot bounds are

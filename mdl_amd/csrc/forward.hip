@@ -792,8 +792,8 @@ __global__ MDL_OCCUPANCY __launch_bounds__(kFwdWaves * kWave) void forward_kerne
 
 // ------------------------------------------------------ pool backward --
 
-// Per-wave LDS of an unpooled chunk: bag bounds relative to the chunk's first
-// position, every bag's divisor with its reciprocal, and the bag of each
+// Per-wave LDS of an unpooled chunk: bag bounds (absolute positions), every
+// bag's divisor with its reciprocal, and the bag of each
 // position of one window (kNoBag: the position's gradient is zero).
 constexpr int kPosWindow = 512;
 constexpr uint16_t kNoBag = 0xffff;

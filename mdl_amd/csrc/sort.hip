@@ -1,7 +1,7 @@
 // Stable LSD radix sort of (uint32 key, uint32 payload) pairs and the
 // torch.unique-style dedup built on it.
 //
-// Each 8-bit pass is three launches:
+// Each pass (a digit of at most 8 bits) is three launches:
 //   upsweep   - per-tile digit histogram  -> counts[digit][tile]
 //   scan      - one block per digit scans its row of counts (tile order)
 //   downsweep - ranks the tile's keys stably, stages them in LDS in digit

@@ -488,7 +488,7 @@ class SequenceStep:
         groups = plan.groups  # row bases of the tables within their key group
         self.device = ids[0].device
         self.ids = [_as_ids(t) for t in ids]
-        self.lengths = [t.to(torch.int64).contiguous() for t in lengths]
+        self.lengths = self._row_lengths(lengths)
         self.all_outputs = [list(o) for o in outputs]
         self.all_masks = [list(m) for m in masks]
         self.all_grads = [[g.contiguous() for g in gs] for gs in grads]
@@ -568,6 +568,17 @@ class SequenceStep:
         self._weights = [t.weight for t in plan.tables]
         self._states = [t.state for t in plan.tables]
 
+    def _row_lengths(self, lengths: Sequence[Tensor]) -> list[Tensor]:
+        # the launches read one length per row at these addresses
+        if len(lengths) != len(self.ids):
+            raise ValueError("one tensor of sequence lengths per feature")
+        for t, x in zip(lengths, self.ids):
+            if t.device != self.device:
+                raise RuntimeError("sequence lengths must live on the step's device")
+            if int(t.numel()) < int(x.size(0)):
+                raise ValueError("sequence lengths must hold one entry per row")
+        return [t.to(torch.int64).contiguous() for t in lengths]
+
     def _n(self, gs: _SeqGroup) -> int:
         return max(gs.cap, 1) * self.k if self.k > 1 else gs.cap
 
@@ -580,7 +591,7 @@ class SequenceStep:
                 raise ValueError("sequence ids must keep their [B, L_in] shapes")
             self.ids = new
         if lengths is not None:
-            new = [t.to(torch.int64).contiguous() for t in lengths]
+            new = self._row_lengths(lengths)
             if [tuple(t.shape) for t in new] != [tuple(t.shape) for t in self.lengths]:
                 raise ValueError("sequence lengths must keep their [B] shapes")
             self.lengths = new
