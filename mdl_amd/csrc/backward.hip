@@ -24,6 +24,7 @@
 #include <mutex>
 
 #include "common.cuh"
+#include "scan.cuh"
 #include "tile_sort.cuh"
 
 namespace mdl {
@@ -484,53 +485,22 @@ __global__ void unique_range_end_kernel(int32_t T, const int64_t* table_start, c
 }
 
 // The scan of the chunks' head counts and the tables' ranges in one block:
-// calls of few chunks would spend a launch on each (two for the scan).
+// calls of few chunks would spend a launch on each (two for the scan; 8.4 us
+// of kernels and two gaps).  8 K chunks take 8 us, 32 K 15.5.
 constexpr int kHeadThreads = 1024;
-constexpr int kHeadItems = 8;
-constexpr int64_t kHeadBlockChunks = 4 * kHeadThreads * kHeadItems;
+constexpr int64_t kHeadBlockChunks = 4 * kHeadThreads * kScanItems;
 
 __global__ __launch_bounds__(kHeadThreads) void heads_range_kernel(
     const int64_t* __restrict__ heads, const int64_t* __restrict__ num_chunks, int64_t max_chunks, int32_t T,
     const int64_t* table_start, const int64_t* table_end, const int64_t* chunk_base, int64_t* head_base,
     const mdl_table* __restrict__ tables, int64_t* unique_range, ChunkRule rule) {
-  __shared__ int32_t s_wave[kHeadThreads / kWave];
+  __shared__ ScanStage<kHeadThreads> st;
   const int64_t m = *num_chunks < max_chunks ? *num_chunks : max_chunks;
-  const int tid = threadIdx.x, w = tid / kWave, lane = lane_id();
-  int64_t carry = 0;
-  if (tid == 0) head_base[0] = 0;
-  for (int64_t base = 0; base < m; base += kHeadThreads * kHeadItems) {
-    const int64_t first = base + (int64_t)tid * kHeadItems;
-    int32_t v[kHeadItems], s = 0;  // (a chunk has at most 512 heads)
-#pragma unroll
-    for (int k = 0; k < kHeadItems; ++k) v[k] = first + k < m ? (int32_t)heads[first + k] : 0;
-#pragma unroll
-    for (int k = 0; k < kHeadItems; ++k) s += v[k];
-    int32_t x = s;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-      const int o = shfl_i(x, lane >= d ? lane - d : lane);
-      if (lane >= d) x += o;
-    }
-    if (lane == kWave - 1) s_wave[w] = x;
-    __syncthreads();
-    int32_t before = 0, all = 0;
-#pragma unroll
-    for (int q = 0; q < kHeadThreads / kWave; ++q) {
-      before += q < w ? s_wave[q] : 0;
-      all += s_wave[q];
-    }
-    int64_t run = carry + before + x - s;
-#pragma unroll
-    for (int k = 0; k < kHeadItems; ++k) {
-      run += v[k];
-      if (first + k < m) head_base[first + k + 1] = run;
-    }
-    carry += all;
-    __syncthreads();  // (also: this block's head_base writes before the reads below)
-  }
+  scan_in_block<kHeadThreads>(heads, m, st, head_base);
+  // this block's head_base writes before the reads below
   __threadfence_block();
   __syncthreads();
-  for (int32_t t = tid; t < T; t += kHeadThreads)
+  for (int32_t t = threadIdx.x; t < T; t += kHeadThreads)
     write_unique_range(t, table_start, table_end, chunk_base, head_base, tables, unique_range, rule);
 }
 

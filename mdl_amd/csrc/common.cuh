@@ -432,6 +432,12 @@ __device__ __forceinline__ uint32_t shfl_u(uint32_t v, int src) {
   return (uint32_t)__builtin_amdgcn_ds_bpermute(src << 2, (int)v);
 }
 
+// Orders a wave's LDS accesses before and after it.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
 // Lanes per row: next power of two >= ceil(dim / C), capped at one wave.
 __host__ __device__ __forceinline__ int lanes_for(int dim, int c) {
   int need = (dim + c - 1) / c;

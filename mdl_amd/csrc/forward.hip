@@ -104,8 +104,6 @@ __device__ __forceinline__ int feat_variant(const Feat& f) {
                     f.dim);
 }
 
-__device__ __forceinline__ void wave_sync() { __builtin_amdgcn_wave_barrier(); __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
-
 template <int C>
 __device__ __forceinline__ void zero_c(float (&v)[C]) {
 #pragma unroll

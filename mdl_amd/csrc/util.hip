@@ -1,5 +1,6 @@
 // Error state, bucketing and the lengths -> offsets scan.
 #include "common.cuh"
+#include "scan.cuh"
 
 #include <cstdio>
 
@@ -84,46 +85,13 @@ static int validate_bucket_mode(const char* who, int32_t mode, int64_t num_bucke
 // ----------------------------------------------------------------- scan --
 
 constexpr int kScanThreads = 256;
-constexpr int kScanItems = 8;
 constexpr int kScanTile = kScanThreads * kScanItems;
-// A scan of up to kScanOneBlock lengths is one block's, in one launch, two
-// rounds of it at most (2.8 us a round and 1 us for the second; the tile sums
-// and the scan of more take 7.2 us at 16 K).
+// A scan of up to kScanOneBlock lengths is one block's, in one launch: for
+// 16384 lengths 7.4 us when they were just written and 8.5 from HBM, for 24576
+// 10.7 and 12.0; the tile sums and the scan of the tiles take 9.3 us with the
+// gap between them for either.
 constexpr int kScanOneThreads = 1024;
-constexpr int kScanOneTile = kScanOneThreads * kScanItems;
-constexpr int kScanOneBlock = 2 * kScanOneTile;
-
-__device__ __forceinline__ int64_t shfl_i64(int64_t v, int src) {
-  const uint32_t lo = (uint32_t)shfl_i((int)(uint32_t)v, src), hi = (uint32_t)shfl_i((int)(v >> 32), src);
-  return (int64_t)(((uint64_t)hi << 32) | lo);
-}
-
-// Exclusive scan of one value per thread over a block of kThreads: shuffles
-// inside each wave, one barrier for the wave totals (256 threads through LDS
-// alone took 16 barriers and half the scan's time).  smem holds a word per
-// wave.
-template <int kThreads>
-__device__ __forceinline__ int64_t block_exclusive_scan(int64_t v, int64_t* smem, int64_t* total) {
-  constexpr int kWaves = kThreads / kWave;
-  const int lane = lane_id(), w = threadIdx.x / kWave;
-  int64_t x = v;
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const int64_t o = shfl_i64(x, lane >= d ? lane - d : lane);
-    if (lane >= d) x += o;
-  }
-  if (lane == kWave - 1) smem[w] = x;
-  __syncthreads();
-  int64_t before = 0, all = 0;
-#pragma unroll
-  for (int q = 0; q < kWaves; ++q) {
-    before += q < w ? smem[q] : 0;
-    all += smem[q];
-  }
-  if (total) *total = all;
-  __syncthreads();
-  return before + x - v;
-}
+constexpr int64_t kScanOneBlock = 2 * kScanOneThreads * kScanItems;
 
 // Sum over a block of kScanThreads, valid in its first thread.
 __device__ __forceinline__ int64_t block_sum_i64(int64_t v, int64_t* smem) {
@@ -136,36 +104,10 @@ __device__ __forceinline__ int64_t block_sum_i64(int64_t v, int64_t* smem) {
   return t;
 }
 
-// offsets[i + 1] = prefix + sum(in[0 .. i]) over this block's tile of
-// blockDim.x * kScanItems lengths from base.
-// Returns the tile's sum.
-template <int kThreads>
-__device__ __forceinline__ int64_t scan_tile(const int64_t* __restrict__ in, int64_t n, int64_t base, int64_t prefix,
-                                             int64_t* smem, int64_t* __restrict__ offsets) {
-  const int64_t first = base + (int64_t)threadIdx.x * kScanItems;
-  int64_t v[kScanItems];
-  int64_t s = 0;
-#pragma unroll
-  for (int k = 0; k < kScanItems; ++k) v[k] = first + k < n ? in[first + k] : 0;
-#pragma unroll
-  for (int k = 0; k < kScanItems; ++k) s += v[k];
-  int64_t all;
-  int64_t ex = block_exclusive_scan<kThreads>(s, smem, &all) + prefix;
-#pragma unroll
-  for (int k = 0; k < kScanItems; ++k) {
-    ex += v[k];
-    if (first + k < n) offsets[first + k + 1] = ex;
-  }
-  return all;
-}
-
 __global__ __launch_bounds__(kScanOneThreads) void scan_one_block(const int64_t* __restrict__ in, int64_t n,
                                                                   int64_t* __restrict__ offsets) {
-  __shared__ int64_t smem[kScanOneThreads / kWave];
-  if (threadIdx.x == 0) offsets[0] = 0;
-  int64_t carry = 0;
-  for (int64_t base = 0; base < n; base += kScanOneTile)
-    carry += scan_tile<kScanOneThreads>(in, n, base, carry, smem, offsets);
+  __shared__ ScanStage<kScanOneThreads> st;
+  scan_in_block<kScanOneThreads>(in, n, st, offsets);
 }
 
 __global__ __launch_bounds__(kScanThreads) void scan_tile_sums(const int64_t* __restrict__ in, int64_t n,
@@ -205,17 +147,20 @@ __global__ __launch_bounds__(kScanThreads) void scan_sums_single(int64_t* __rest
 __global__ __launch_bounds__(kScanThreads) void scan_tiles_final(const int64_t* __restrict__ in, int64_t n,
                                                                  const int64_t* __restrict__ sums,
                                                                  int64_t* __restrict__ offsets, int prefix_self) {
-  __shared__ int64_t smem[kScanThreads / kWave];
+  __shared__ ScanStage<kScanThreads> st;
   int64_t tile_prefix;
   if (prefix_self) {
     int64_t p = 0;
     for (int64_t j = threadIdx.x; j < (int64_t)blockIdx.x; j += kScanThreads) p += sums[j];
-    block_exclusive_scan<kScanThreads>(p, smem, &tile_prefix);
+    block_exclusive_scan<kScanThreads>(p, st.wave, &tile_prefix);
   } else {
     tile_prefix = sums[blockIdx.x];
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) offsets[0] = 0;
-  scan_tile<kScanThreads>(in, n, (int64_t)blockIdx.x * kScanTile, tile_prefix, smem, offsets);
+  const int64_t base = (int64_t)blockIdx.x * kScanTile;
+  int64_t v[kScanItems];
+  load_scan_tile<kScanThreads>(in, n, base, v);
+  scan_tile<kScanThreads>(v, n, base, tile_prefix, st, offsets);
 }
 
 // ------------------------------------------------------ list truncation --

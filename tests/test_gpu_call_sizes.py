@@ -27,6 +27,52 @@ def test_offsets_scan(device, n):
     assert np.array_equal(got, np.concatenate([[0], np.cumsum(ln)]))
 
 
+@pytest.mark.parametrize("n", [2, 3, 63, 2047, 2048, 2049, 2050, 4095, 8193 + 511, 24577])
+def test_offsets_scan_of_one_block_and_of_tiles(device, n):
+    """Lengths two a thread (2048 at most), eight a thread through LDS, and a
+    second tile of one that ends inside a wave; the last offset alone when
+    the lengths before it are zeros."""
+
+    print("CASE scan places", n, flush=True)
+    rng = np.random.default_rng(n)
+    for ln in (rng.integers(-5, 1 << 40, size=n), np.eye(1, n, n - 1, dtype=np.int64)[0]):
+        got = ops.lengths_to_offsets(torch.from_numpy(ln).to(device)).cpu().numpy()
+        assert np.array_equal(got, np.concatenate([[0], np.cumsum(ln)]))
+
+
+@pytest.mark.parametrize("dim, n", [(64, 9000), (256, 40000), (256, 150000), (256, 500000), (256, 600000)])
+def test_distinct_rows_of_many_chunks(device, dim, n):
+    """The distinct rows of several tables where their chunks' head counts are
+    scanned two a thread, in one tile, in several and by launches of tiles."""
+
+    print("CASE heads", dim, n, flush=True)
+    rng = np.random.default_rng(n)
+    rows = [1, 70000, 5, 400000]
+    tables = np.zeros(len(rows), dtype=_lib.TABLE_DTYPE)
+    tables["row_base"] = np.concatenate([[0], np.cumsum(rows)[:-1]])
+    tables["num_rows"] = rows
+    tables["dim"] = dim
+    tables["feature"] = -1
+    total = sum(rows)
+    keys = rng.integers(0, total + total // 50, size=n)
+    keys = np.minimum(keys, total).astype(np.uint32)
+    L = _lib.lib()
+    tdev = torch.from_numpy(tables.view(np.uint8)).to(device)
+    k = torch.from_numpy(keys.view(np.int32).copy()).to(device)
+    p = torch.arange(n, dtype=torch.int32, device=device)
+    ws = torch.empty(int(L.mdl_backward_workspace_bytes(n, len(rows), dim)), dtype=torch.uint8, device=device)
+    urange = torch.full((2 * len(rows),), -1, dtype=torch.int64, device=device)
+    _lib.check(L.mdl_backward_count(
+        tdev.data_ptr(), len(rows), dim, k.data_ptr(), p.data_ptr(), n, None, total.bit_length(), urange.data_ptr(),
+        ws.data_ptr(), ws.numel(), torch.cuda.current_stream(device).cuda_stream), "mdl_backward_count")
+    ur = urange.cpu().numpy().reshape(-1, 2)
+    uniq = np.unique(keys)
+    lo = tables["row_base"]
+    below = np.searchsorted(uniq, lo)
+    assert np.array_equal(ur[:, 0], below)
+    assert np.array_equal(ur[:, 1], np.searchsorted(uniq, lo + tables["num_rows"]))
+
+
 @pytest.mark.parametrize("rows", [1, 255, 256, 257, 2049])
 @pytest.mark.parametrize("longest", [0, 3, 1200])
 @pytest.mark.parametrize("truncation", ["head", "tail"])
