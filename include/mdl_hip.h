@@ -452,7 +452,10 @@ int mdl_backward_apply(const mdl_feature* feats, int32_t num_features,
  * one stretch (a grouped lookup whose tables are read by one feature each),
  * short enough that sorting tiles and merging those that overlap beats the
  * radix passes.  mdl_sort_hints says so from each table's entry count (a
- * host array; the counts of a typical batch do).
+ * host array; the counts of a typical batch do).  A call with a device count
+ * takes the hint as another batch's and follows it up to 128 tiles of 4096
+ * entries (n, its capacity): a batch gathered in one table then costs the sort
+ * at most 0.13 ms more.
  */
 #define MDL_SORT_BY_TABLE 1u
 uint32_t mdl_sort_hints(const int64_t* table_entries, int32_t num_tables);

@@ -1258,17 +1258,28 @@ static int plan(const mdl_table* tables, int32_t T, const uint32_t* sk, int64_t 
 //   pair overlapping) 38 -> 30; 393 K of 32 tables 59 -> 31; 131 K of 8 tables
 //   50 -> 32; 893 K of 64 tables, 24 of 34 K, 58 -> 51; 3.3 M of 200 tables of
 //   16 K 117 -> 98.
-// A merge costs about 1 us per two overlapping tiles, so entries in an order
-// the call does not know merge up to kMergeFreeTiles tiles; a call hinted to
-// come table by table has every table short enough (mdl_sort_hints): at
-// kHintLongest tiles a table, or kHintPairs overlapping pairs in all, the two
-// sorts take about the same time.
+// A merge costs a round of about 1 us per two overlapping tiles, and its
+// blocks are all in flight up to some 250 tiles, so entries in an order the
+// call does not know merge up to kMergeFreeTiles tiles, and a call hinted to
+// come table by table has every table short enough (mdl_sort_hints).  The two
+// sorts take about the same time at kHintLongest tiles a table, or where
+// kHintOverlaps times a tile meets another of its table (radix -> tiles:
+// tables of 9 tiles, 28 of them 55 -> 49 us, 48 78 -> 75, 56 76 -> 82, 113
+// 95 -> 145; of 7, 64 77 -> 68, 90 84 -> 91; of 5, 150 98 -> 86, 200 110 ->
+// 106; of 2, 500 117 -> 93; of 8, 50 69 -> 72, 100 90 -> 123).
+// A call that takes its entry count from the device was hinted from another
+// batch's counts.  With every entry in one table all its tiles meet: 96
+// tiles 50 -> 145 us, 127 53 -> 186, 218 64 -> 546, 1024 108 -> 9033 (spread over
+// 64 tables 51 -> 24, 53 -> 32, 65 -> 43, 107 -> 214).  So such calls merge up to
+// kCountedTiles tiles.
 constexpr int64_t kMergeFreeTiles = 12;
-constexpr int64_t kHintLongest = 10, kHintPairs = 16384;
-static bool sorts_by_tiles(int64_t n, int32_t key_bits, uint32_t hints) {
+constexpr int64_t kHintLongest = 10, kHintOverlaps = 4500;
+constexpr int64_t kCountedTiles = 128;
+static bool sorts_by_tiles(int64_t n, int32_t key_bits, uint32_t hints, bool counted) {
   if (key_bits <= 0 || key_bits > 32) return false;
   const int64_t tiles = merge_tiles(n);
-  return tiles <= kMergeFreeTiles || ((hints & MDL_SORT_BY_TABLE) && tiles <= kMaxMergeTiles);
+  return tiles <= kMergeFreeTiles ||
+         ((hints & MDL_SORT_BY_TABLE) && tiles <= (counted ? kCountedTiles : kMaxMergeTiles));
 }
 
 static int prepare(const mdl_table* tables, int32_t T, int32_t max_dim, uint32_t* keys, uint32_t* payload,
@@ -1276,7 +1287,7 @@ static int prepare(const mdl_table* tables, int32_t T, int32_t max_dim, uint32_t
                    hipStream_t s, BwdWs* w, const uint32_t** sk, const uint32_t** sv) {
   const size_t need = carve(w, ws, n, T, max_dim);
   if (ws_bytes < need) return fail(MDL_ERR_WORKSPACE, "backward: workspace too small");
-  if (sorts_by_tiles(n, key_bits, hints)) {
+  if (sorts_by_tiles(n, key_bits, hints, n_dev != nullptr)) {
     // The sorted pairs end where the radix passes would leave them (the
     // calls that follow the sort derive that from key_bits).
     const bool in_alt = sort_pass_count(key_bits) & 1;
@@ -1526,13 +1537,13 @@ size_t mdl_backward_workspace_bytes(int64_t n, int32_t num_tables, int32_t max_d
 }
 
 uint32_t mdl_sort_hints(const int64_t* table_entries, int32_t num_tables) {
-  int64_t pairs = 0, longest = 0;
+  int64_t overlaps = 0, longest = 0;
   for (int32_t t = 0; t < num_tables; ++t) {
     const int64_t tiles = merge_tiles(table_entries[t]) + 1;  // a stretch starts anywhere in a tile
     longest = tiles > longest ? tiles : longest;
-    pairs += tiles * tiles;
+    overlaps += tiles * (tiles - 1);
   }
-  return longest <= kHintLongest && pairs <= kHintPairs ? MDL_SORT_BY_TABLE : 0u;
+  return longest <= kHintLongest && overlaps <= kHintOverlaps ? MDL_SORT_BY_TABLE : 0u;
 }
 
 int mdl_backward_sort_hinted(const mdl_table* tables, int32_t num_tables, int32_t max_dim, uint32_t* sort_keys,

@@ -82,7 +82,10 @@ class SparseStep:
     None when no feature is pooled; ``id_counts`` / ``bag_counts``: per
     feature, for this first batch (they size the chunks; bag counts are the
     batch size of each pooled feature and stay fixed, and so does the id count
-    of an unpooled feature, one per output row).  ``capacity`` bounds the ids
+    of an unpooled feature, one per output row).  They also choose the
+    backward's sort; batches whose ids gather in fewer tables give the same
+    result, up to 128 tiles of 4096 ids in a slower sort
+    (``mdl_backward_sort_hinted``).  ``capacity`` bounds the ids
     of any batch bound later (default: this batch's).  Outputs and gradients
     are 2-D row views (e.g. column slices of one ``[B, sum(dim)]`` buffer).
 

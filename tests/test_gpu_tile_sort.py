@@ -93,3 +93,51 @@ def test_sort_hints_follow_the_stretches():
     assert hints([4096 * 9]) == 1
     assert hints([4096 * 9 + 1]) == 0
     assert hints([4096 * 9] * 200) == 0
+
+
+def test_sort_hints_stop_where_the_radix_sort_is_faster():
+    """Tables of several tiles each, many of them: every tile meets the others
+    of its table, and the merge's blocks no longer run all at once."""
+
+    def hints(counts):
+        c = np.asarray(counts, dtype=np.int64)
+        return int(_lib.lib().mdl_sort_hints(c.ctypes.data, len(c)))
+
+    assert hints([TILE * 9] * 28) == 1
+    assert hints([TILE * 9] * 56) == 0
+    assert hints([TILE * 8] * 100) == 0
+    assert hints([TILE * 4] * 200) == 1
+    assert hints([TILE] * 1000) == 1
+
+
+@pytest.mark.parametrize("tiles, counted, merges", [(128, True, True), (129, True, False), (129, False, True)])
+def test_hint_of_another_batch_is_followed_up_to_a_bound(device, tiles, counted, merges):
+    """A call with a device count was hinted from another batch, whose tables
+    this one's ids may not spread over: past 128 tiles it takes the radix
+    passes, whose time does not depend on that."""
+
+    n, rows = tiles * TILE - 3, 1 << 20
+    print("CASE hint bound", tiles, counted, flush=True)
+    tables = np.zeros(64, dtype=_lib.TABLE_DTYPE)
+    tables["row_base"] = np.arange(64) * rows
+    tables["num_rows"] = rows
+    tables["dim"] = 16
+    tables["feature"] = -1
+    keys = np.random.default_rng(tiles).integers(0, rows, size=n).astype(np.uint32)  # one table's
+    tdev = torch.from_numpy(tables.view(np.uint8)).to(device)
+    k = torch.from_numpy(keys.view(np.int32).copy()).to(device)
+    p = torch.arange(n, dtype=torch.int32, device=device)
+    count = torch.tensor([n], dtype=torch.int64, device=device)
+    L = _lib.lib()
+    ws = torch.empty(int(L.mdl_backward_workspace_bytes(n, 64, 16)), dtype=torch.uint8, device=device)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        _lib.check(L.mdl_backward_sort_hinted(
+            tdev.data_ptr(), 64, 16, k.data_ptr(), p.data_ptr(), n, count.data_ptr() if counted else None, 32, 1,
+            ws.data_ptr(), ws.numel(), torch.cuda.current_stream(device).cuda_stream), "mdl_backward_sort_hinted")
+        torch.cuda.synchronize()
+    names = " ".join(e.key for e in prof.key_averages())
+    assert ("rank_merge_kernel" in names) == merges
+    assert ("radix_downsweep" in names) != merges
+    want = np.argsort(keys, kind="stable")
+    assert np.array_equal(p.cpu().numpy(), want)
+    assert np.array_equal(k.cpu().numpy().view(np.uint32), keys[want])
