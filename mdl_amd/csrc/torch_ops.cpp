@@ -2182,16 +2182,15 @@ TORCH_LIBRARY(mdl_hip, m) {
         "int max_dim, int key_bits, int classes, float max_norm=0., Tensor(c!)? total_norm=None, "
         "Tensor(d!)? coef=None) -> ()",
         &backward_sumsq_);
+  // Per-backend kernels below, none for tensors without data: what traces
+  // calls with fake or functional tensors must not reach a launch.
   m.def("bag_truncate_exact(Tensor values, Tensor offsets, Tensor? valid, Tensor? row_valid, int max_length, "
-        "str truncation, str bucket, int num_buckets, bool validate_nonzero) -> (Tensor, Tensor, int)",
-        &bag_truncate_exact);
+        "str truncation, str bucket, int num_buckets, bool validate_nonzero) -> (Tensor, Tensor, int)");
   // Pooling of already-embedded rows (mdl_amd/pooling.py's autograd function).
   m.def("pool_bags_forward(Tensor[] embedded, Tensor[] ids, Tensor[] lengths, int[] codes, bool mean, "
-        "Tensor(a!)? counter) -> (Tensor[], Tensor, Tensor, Tensor)",
-        &pool_bags_forward);
+        "Tensor(a!)? counter) -> (Tensor[], Tensor, Tensor, Tensor)");
   m.def("pool_bags_backward(Tensor[] grads, int[] needs, int[] rows, int[] dims, int[] batches, int[] codes, "
-        "bool mean, Tensor ids, Tensor offsets, Tensor bag_count) -> Tensor[]",
-        &pool_bags_backward);
+        "bool mean, Tensor ids, Tensor offsets, Tensor bag_count) -> Tensor[]");
   m.def("clip_coefficient_(Tensor sumsq, int count, float max_norm, Tensor(a!) total_norm, Tensor(b!) coef) -> ()",
         &clip_coefficient_);
   // The trainer's sparse clip over parameter lists (their gradients scaled
@@ -2213,4 +2212,15 @@ TORCH_LIBRARY_IMPL(mdl_hip, CUDA, m) {
   m.impl("sparse_coalesce_padded", &sparse_coalesce_padded_cuda);
   m.impl("rowwise_adagrad_", &rowwise_adagrad_cuda);
   m.impl("grouped_rowwise_adagrad_", &grouped_rowwise_adagrad_cuda);
+  m.impl("bag_truncate_exact", &bag_truncate_exact);
+  m.impl("pool_bags_forward", &pool_bags_forward);
+  m.impl("pool_bags_backward", &pool_bags_backward);
+}
+
+// (these say in their own words that CPU tensors are not theirs)
+TORCH_LIBRARY_IMPL(mdl_hip, CPU, m) {
+  using namespace mdl_torch;
+  m.impl("bag_truncate_exact", &bag_truncate_exact);
+  m.impl("pool_bags_forward", &pool_bags_forward);
+  m.impl("pool_bags_backward", &pool_bags_backward);
 }

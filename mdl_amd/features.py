@@ -144,8 +144,10 @@ def bag_csr_tensor(
         raise ValueError("pre_hashed num_buckets must be a positive power of two")
     args = (values, offsets, valid, row_valid, -1 if max_length is None else int(max_length), truncation, bucket,
             int(num_buckets), bool(validate_nonzero))
-    if exact and values.is_cuda and type(values) is Tensor and not torch.compiler.is_compiling():
-        # one call, its two numbers read back together
+    if (exact and values.is_cuda and type(values) is Tensor and not torch.compiler.is_compiling()
+            and torch._C._len_torch_dispatch_stack() == 0):
+        # one call, its two numbers read back together (a tracer sees the
+        # general call, whose total is data)
         ids, lengths, bad = torch.ops.mdl_hip.bag_truncate_exact(*args)
         total = ids.numel()
     else:

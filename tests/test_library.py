@@ -397,6 +397,59 @@ def test_frozen_table_in_a_grouped_lookup_gets_no_gradient(device):
     assert dense[1].tolist() == [1.0] * 4 and dense[2].tolist() == [2.0] * 4 and float(dense.abs().sum()) == 12.0
 
 
+def test_ops_without_a_fake_kernel_refuse_tensors_without_data():
+    """A tracer's fake tensors have no memory: these operators end in the
+    dispatcher for them, before anything is launched on their addresses."""
+
+    from torch._subclasses import FakeTensorMode
+    from torch._subclasses.fake_tensor import UnsupportedOperatorException
+
+    with FakeTensorMode():
+        rows, grad, counts = (torch.empty(n, 4, device="cuda") for n in (6, 3, 3))
+        ids, ln, off = (torch.empty(n, dtype=torch.int64, device="cuda") for n in (6, 3, 4))
+        with pytest.raises(UnsupportedOperatorException):
+            OPS.pool_bags_forward([rows], [ids], [ln], [0], True, None)
+        with pytest.raises(UnsupportedOperatorException):
+            OPS.pool_bags_backward([grad], [1], [6], [4], [3], [0], True, ids, off, counts[:, 0])
+        with pytest.raises(UnsupportedOperatorException):
+            OPS.bag_truncate_exact(ids, off, None, None, 2, "head", "none", 0, False)
+
+
+@pytest.mark.gpu
+def test_pooling_and_list_encoding_around_a_tracer():
+    """torch.compile runs pool_bags outside its graphs with the eager results
+    and gradients; a traced bag_csr_tensor(exact=True) is refused as data
+    dependent, compiled it gives the eager lists."""
+
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    from mdl_amd.features import bag_csr_tensor
+    from mdl_amd.pooling import pool_bags
+
+    ids, ln = torch.tensor([1, 0, 2, 3, 4, 5], device="cuda"), torch.tensor([2, 0, 4], device="cuda")
+
+    def pool(e):
+        a, b = pool_bags([(e * 2, ids, ln, "exclude"), (e + 1, ids, ln, "include_as_padding")])
+        return a.sum() + (b * 3).square().sum()
+
+    grads = []
+    for fn in (pool, torch.compile(pool, backend="aot_eager")):
+        e = torch.arange(24, dtype=torch.float32, device="cuda").view(6, 4).requires_grad_()
+        fn(e).backward()
+        grads.append(e.grad)
+    assert torch.equal(*grads)
+
+    def encode(v, o):
+        got = bag_csr_tensor(v + 1, o, max_length=2, exact=True)
+        return got["values"], got["lengths"]
+
+    args = torch.arange(6, device="cuda"), torch.tensor([0, 3, 6], device="cuda")
+    for got, want in zip(torch.compile(encode, backend="aot_eager")(*args), encode(*args)):
+        assert torch.equal(got, want)
+    with pytest.raises(RuntimeError):
+        make_fx(encode)(*args)
+
+
 def test_modules_compile_with_their_gradients(capacity_grads):
     """torch.compile (full graph, AOT autograd) traces the modules' lookups:
     fake tensors take the op's registered autograd, and the compiled step's
