@@ -397,6 +397,42 @@ def test_frozen_table_in_a_grouped_lookup_gets_no_gradient(device):
     assert dense[1].tolist() == [1.0] * 4 and dense[2].tolist() == [2.0] * 4 and float(dense.abs().sum()) == 12.0
 
 
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("reached", [[0], [1], [2, 4], [3], [0, 1, 3]])
+def test_outputs_the_loss_does_not_reach(device, dtype, reached):
+    """A loss over some of a lookup's outputs gives every table the gradient
+    that explicit zeros for the others give: bags, 1-D and 2-D ids, two
+    features of one table, and a sequence whose mask and count have none."""
+
+    dims = [("a", 20, 4), ("b", 20, 8), ("c", 30, 16)]
+
+    def run(explicit):
+        torch.manual_seed(1)
+        a, b, c = (m.to(device, dt) for m, dt in zip(_modules(dims), (torch.float32, dtype, torch.bfloat16)))
+        outs = grouped_sharded_embedding_lookup([
+            (a, torch.tensor([1, 2, 2], device=device)), (b, torch.tensor([[3, 4, 4], [0, 1, 3]], device=device))])
+        ids, ln = torch.tensor([1, 5, 5, 9, 0], device=device), torch.tensor([2, 0, 3], device=device)
+        outs += pooled_embedding_lookup([(c, ids, ln, "mean", "exclude"),
+                                         (a, ids[:3], torch.tensor([3], device=device), "sum", "include_as_padding")])
+        outs.append(sequence_embedding_lookup(b, torch.tensor([[3, 1, 0], [4, 4, 2]], device=device),
+                                              torch.tensor([2, 3], device=device), target_length=4)[0])
+        gen = torch.Generator().manual_seed(2)
+        grads = [torch.randn(o.shape, generator=gen).to(device, o.dtype) for o in outs]
+        if explicit:
+            grads = [g if k in reached else torch.zeros_like(g) for k, g in enumerate(grads)]
+            torch.autograd.backward(outs, grads)
+        else:
+            torch.autograd.backward([outs[k] for k in reached], [grads[k] for k in reached])
+        return [None if m.weight.grad is None else m.weight.grad.to_dense() for m in (a, b, c)]
+
+    for got, want in zip(run(False), run(True)):
+        if got is None:  # none of the table's calls was reached
+            assert not want.any()
+        else:
+            assert torch.equal(got, want)
+
+
 def test_ops_without_a_fake_kernel_refuse_tensors_without_data():
     """A tracer's fake tensors have no memory: these operators end in the
     dispatcher for them, before anything is launched on their addresses."""
