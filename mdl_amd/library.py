@@ -559,13 +559,15 @@ def _sequence_backward(ctx, grad_out, *_unused):
     if grad_out is None:
         grad_out = torch.zeros((ids.size(0), out_len, weight.size(1)), dtype=weight.dtype, device=weight.device)
     # an exact gradient views the live rows only: nothing past them is filled
+    # (the mode is read once: another thread may set it)
     eager = _eager(keys)
+    exact = _grad_mode == "coalesced"
     rows, values, count = torch.ops.mdl_hip.sequence_lookup_backward(
         weight, ids, lengths, out_len, newest_first, padding_idx, grad_out.contiguous(), keys, payload,
-        not (eager and _grad_mode == "coalesced"),
+        not (eager and exact),
     )
     if eager:
-        g = torch.ops.mdl_hip.capacity_sparse_grad(weight, rows, values, count, _grad_mode == "coalesced")
+        g = torch.ops.mdl_hip.capacity_sparse_grad(weight, rows, values, count, exact)
     else:
         g = torch.sparse_coo_tensor(rows.unsqueeze(0), values, tuple(weight.shape), is_coalesced=False)
     return g, None, None, None, None, None, None

@@ -433,6 +433,38 @@ def test_outputs_the_loss_does_not_reach(device, dtype, reached):
             assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("first", ["coalesced", "capacity"])
+def test_a_sequence_backward_keeps_the_gradient_mode_it_began_with(first):
+    """The mode set by another thread while a sequence's backward runs: a
+    gradient whose padding rows were not filled never shows them."""
+
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    mode = mdl_amd.library.sparse_grad_mode()
+    pads = []
+
+    class Flip(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            out = func(*args, **(kwargs or {}))
+            if func is OPS.sequence_lookup_backward.default:
+                # (schema defaults are left off the call)
+                pads.append(args[9] if len(args) > 9 else True)
+                mdl_amd.library.set_sparse_grad_mode("capacity" if first == "coalesced" else "coalesced")
+            return out
+
+    try:
+        (a,) = _modules([("a", 20, 4)])
+        out, _ = sequence_embedding_lookup(a, torch.tensor([[3, 1, 0], [4, 4, 2]]), torch.tensor([2, 3]))
+        mdl_amd.library.set_sparse_grad_mode(first)
+        with Flip():
+            out.sum().backward()
+    finally:
+        mdl_amd.library.set_sparse_grad_mode(mode)
+    distinct = 4
+    assert pads == [first == "capacity"]
+    assert a.weight.grad._nnz() == (distinct if first == "coalesced" else 6)
+
+
 def test_ops_without_a_fake_kernel_refuse_tensors_without_data():
     """A tracer's fake tensors have no memory: these operators end in the
     dispatcher for them, before anything is launched on their addresses."""
