@@ -80,6 +80,49 @@ def test_tile_sort_matches_stable_sort(device, order, rows):
                 assert np.array_equal(ur[:, 1] - ur[:, 0], distinct)
 
 
+@pytest.mark.parametrize("tiles, extra, counted", [
+    (100, 0, True), (128, 0, True), (127, 77, True), (100, 5, False), (512, 0, False), (512, 1, False),
+    (1024, 0, False), (1024, 1, False),
+])
+@pytest.mark.parametrize("order", ["by table", "any"])
+def test_tile_sort_of_many_tiles(device, order, tiles, extra, counted):
+    """Hinted calls up to the bound with a device count (the count at, below
+    and far below the capacity), and without one up to 1024 tiles, where the
+    radix passes take over: more tiles than a block has threads, and, in no
+    order, every tile in a block's list of those that overlap."""
+
+    n, rows = tiles * TILE + extra, [50000] * 63 + [7]
+    rng = np.random.default_rng(tiles + extra)
+    T = len(rows)
+    tables = np.zeros(T, dtype=_lib.TABLE_DTYPE)
+    tables["row_base"] = np.concatenate([[0], np.cumsum(rows)[:-1]])
+    tables["num_rows"] = rows
+    tables["dim"] = 64
+    tables["feature"] = -1
+    tdev = torch.from_numpy(tables.view(np.uint8)).to(device)
+    keys, total = _keys(rng, order, n, rows)
+    L = _lib.lib()
+    ws = torch.empty(int(L.mdl_backward_workspace_bytes(n, T, 64)), dtype=torch.uint8, device=device)
+    for present in ([n, n - TILE - 3, n // 40] if counted else [n]):
+        print("CASE many tiles", order, n, present, flush=True)
+        k = torch.from_numpy(keys.view(np.int32).copy()).to(device)
+        p = torch.arange(n, dtype=torch.int32, device=device)
+        count = torch.tensor([present], dtype=torch.int64, device=device)
+        urange = torch.full((2 * T,), -1, dtype=torch.int64, device=device)
+        _lib.check(L.mdl_backward_count_hinted(
+            tdev.data_ptr(), T, 64, k.data_ptr(), p.data_ptr(), n, count.data_ptr() if counted else None, 32, 1,
+            urange.data_ptr(), ws.data_ptr(), ws.numel(), torch.cuda.current_stream(device).cuda_stream),
+            "mdl_backward_count_hinted")
+        want = np.argsort(keys[:present], kind="stable")
+        assert np.array_equal(p.cpu().numpy()[:present], want)
+        assert np.array_equal(k.cpu().numpy().view(np.uint32)[:present], keys[:present][want])
+        uniq = np.unique(keys[:present])
+        lo = tables["row_base"]
+        ur = urange.cpu().numpy().reshape(T, 2)
+        assert np.array_equal(ur[:, 0], np.searchsorted(uniq, lo))
+        assert np.array_equal(ur[:, 1], np.searchsorted(uniq, lo + tables["num_rows"]))
+
+
 def test_sort_hints_follow_the_stretches():
     """One short stretch per table takes the tile sort; one long one, or
     stretches of too many tile pairs together, the radix sort."""
