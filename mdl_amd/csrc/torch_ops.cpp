@@ -2098,17 +2098,6 @@ void backward_sumsq_(const Tensor& features, int64_t num_features, const Tensor&
         "mdl_backward_sumsq");
 }
 
-void clip_coefficient_(const Tensor& sumsq, int64_t count, double max_norm, const Tensor& total_norm,
-                       const Tensor& coef) {
-  const at::Device dev = sumsq.device();
-  const c10::DeviceGuard guard(dev);
-  TORCH_CHECK_VALUE(sumsq.scalar_type() == at::kFloat && sumsq.is_contiguous() && sumsq.numel() >= count,
-                    "squared norms are a contiguous float32 tensor");
-  check(mdl_clip_coef(sumsq.data_ptr<float>(), (int32_t)count, (float)max_norm, total_norm.data_ptr<float>(),
-                      coef.data_ptr<float>(), stream_of(dev)),
-        "mdl_clip_coef");
-}
-
 }  // namespace mdl_torch
 
 // ---------------------------------------------------------- registration --
@@ -2191,8 +2180,6 @@ TORCH_LIBRARY(mdl_hip, m) {
         "Tensor(a!)? counter) -> (Tensor[], Tensor, Tensor, Tensor)");
   m.def("pool_bags_backward(Tensor[] grads, int[] needs, int[] rows, int[] dims, int[] batches, int[] codes, "
         "bool mean, Tensor ids, Tensor offsets, Tensor bag_count) -> Tensor[]");
-  m.def("clip_coefficient_(Tensor sumsq, int count, float max_norm, Tensor(a!) total_norm, Tensor(b!) coef) -> ()",
-        &clip_coefficient_);
   // The trainer's sparse clip over parameter lists (their gradients scaled
   // in place, some coalesced and stored back).
   m.def("clip_sparse_grad_norm_(Tensor(a!)[] replicated, Tensor(b!)[] sharded, float max_norm) -> Tensor",

@@ -24,7 +24,6 @@ from ._lib import (
     MDL_BF16,
     MDL_F32,
     MDL_FLAG_EXCLUDE_NULL,
-    MDL_FLAG_ROWS_BY_POSITION,
     MDL_POOL_MEAN,
     MDL_POOL_NONE,
     MDL_POOL_SUM,
@@ -329,7 +328,6 @@ class FeatureSpec:
     exclude_null: bool
     padding_idx: int
     out_dtype: torch.dtype
-    rows_by_position: bool = False
 
 
 # Sort keys are 32-bit: the rows of one key group stay below this, and a key
@@ -389,9 +387,9 @@ class GroupPlan:
         # layout when the plan comes from ``memoized_plan``.
         self._memo: dict | None = None
 
-    def add_table(self, weight: Tensor, state: Tensor | None = None, *, shared: bool = True) -> int:
+    def add_table(self, weight: Tensor, state: Tensor | None = None) -> int:
         key = weight.data_ptr()
-        if shared and key in self._table_of_ptr:
+        if key in self._table_of_ptr:
             t = self._table_of_ptr[key]
             if state is not None and self.tables[t].state is None:
                 self.tables[t].state = state
@@ -402,8 +400,7 @@ class GroupPlan:
         _require_device(weight, "embedding weight")
         t = len(self.tables)
         self.tables.append(TableSpec(weight=weight, state=state, row_base=self.total_rows))
-        if shared:
-            self._table_of_ptr[key] = t
+        self._table_of_ptr[key] = t
         if int(weight.size(0)) >= KEY_SPACE:
             raise ValueError("a table of a grouped lookup holds fewer than 2^32 - 1 rows")
         self.total_rows += int(weight.size(0))
@@ -418,19 +415,14 @@ class GroupPlan:
         padding_idx: int = 0,
         state: Tensor | None = None,
         out_dtype: torch.dtype | None = None,
-        rows_by_position: bool = False,
     ) -> int:
-        """Add one lookup request; ``rows_by_position`` pools the rows of an
-        already-embedded ``weight`` (row i = id slot i) instead of looking up
-        ids, which then only decide the null weights."""
+        """Add one lookup request."""
 
         if pooling not in POOLING_CODES:
             raise ValueError(f"unsupported pooling {pooling!r}")
         if null_policy not in NULL_POLICIES:
             raise ValueError(f"unsupported categorical bag null policy {null_policy!r}")
-        if rows_by_position and pooling == "none":
-            raise ValueError("rows by position need a pooled feature")
-        t = self.add_table(weight, state, shared=not rows_by_position)
+        t = self.add_table(weight, state)
         self.features.append(
             FeatureSpec(
                 table=t,
@@ -438,7 +430,6 @@ class GroupPlan:
                 exclude_null=null_policy == "exclude",
                 padding_idx=int(padding_idx),
                 out_dtype=out_dtype or weight.dtype,
-                rows_by_position=bool(rows_by_position),
             )
         )
         return len(self.features) - 1
@@ -499,7 +490,7 @@ class GroupPlan:
             for spec in self.features[lo:hi]:
                 sub.features.append(FeatureSpec(
                     table=local[spec.table], pooling=spec.pooling, exclude_null=spec.exclude_null,
-                    padding_idx=spec.padding_idx, out_dtype=spec.out_dtype, rows_by_position=spec.rows_by_position,
+                    padding_idx=spec.padding_idx, out_dtype=spec.out_dtype,
                 ))
             groups.append(KeyGroup(lo, hi, tabs, rows, sub))
         return groups
@@ -583,10 +574,7 @@ def _static_features(plan: GroupPlan) -> np.ndarray:
     feats["wdtype"] = [dtype_code(t.weight.dtype) for t in tab]
     feats["odtype"] = [dtype_code(s.out_dtype) for s in specs]
     feats["pooling"] = np.array([s.pooling for s in specs], dtype=np.int32)
-    feats["flags"] = [
-        (MDL_FLAG_EXCLUDE_NULL if s.exclude_null else 0) | (MDL_FLAG_ROWS_BY_POSITION if s.rows_by_position else 0)
-        for s in specs
-    ]
+    feats["flags"] = [MDL_FLAG_EXCLUDE_NULL if s.exclude_null else 0 for s in specs]
     feats["padding_idx"] = [s.padding_idx for s in specs]
     feats["table"] = [s.table for s in specs]
     for s, t in zip(specs, tab):
@@ -648,7 +636,6 @@ def forward_packed(
     *,
     with_backward: bool,
     error_count: Tensor | None = None,
-    with_bag_count: bool | None = None,
 ) -> ForwardResult:
     """Grouped lookup over caller-packed buffers (no per-feature copies).
 
@@ -656,8 +643,7 @@ def forward_packed(
     bounds from one scan of the concatenated lengths (see build_features);
     ``outputs[f]``: row-major output rows of feature f (2-D views with unit
     column stride, e.g. column slices of one ``[B, sum(dim)]`` buffer).
-    ``with_backward`` emits the backward's sort keys and bag counts;
-    ``with_bag_count`` (default: ``with_backward``) only the bag counts.
+    ``with_backward`` emits the backward's sort keys and bag counts.
     """
 
     device = all_ids.device
@@ -684,13 +670,11 @@ def forward_packed(
         error_count = torch.zeros(1, dtype=torch.int32, device=device)
     keys = payload = bag_count = None
     total_rows_out = int(feats["payload_base"][-1] + (feats["num_bags"][-1] if feats["pooling"][-1] else feats["num_ids"][-1])) if len(feats) else 0
-    if with_bag_count is None:
-        with_bag_count = with_backward
     if with_backward:
         alloc = torch.empty if n else torch.zeros
         keys = alloc(max(n, 1), dtype=torch.int32, device=device)
         payload = alloc(max(n, 1), dtype=torch.int32, device=device)
-    if with_bag_count and pooled_any:
+    if with_backward and pooled_any:
         # zeros: the rows of unpooled features have no bag and are not written
         bag_count = torch.zeros(max(total_rows_out, 1), dtype=torch.float32, device=device)
     check(
@@ -716,7 +700,6 @@ def grouped_forward(
     with_backward: bool,
     outputs: Sequence[Tensor] | None = None,
     error_count: Tensor | None = None,
-    with_bag_count: bool | None = None,
 ) -> ForwardResult:
     """Look up (and pool) every feature of ``plan`` in one launch.
 
@@ -777,7 +760,7 @@ def grouped_forward(
                 raise ValueError("caller outputs must have unit column stride and the feature's dtype")
     return forward_packed(
         plan, all_ids, offsets, id_counts, bag_counts, outputs,
-        with_backward=with_backward, error_count=error_count, with_bag_count=with_bag_count,
+        with_backward=with_backward, error_count=error_count,
     )
 
 
@@ -884,67 +867,6 @@ def _attach_grads(res: ForwardResult, grads: Sequence[Tensor | None]) -> tuple[n
     feats["grad"] = np.asarray(gptr, dtype=np.uint64)
     feats["out_stride"] = np.asarray(gstride, dtype=np.int64)
     return feats, keep
-
-
-def pool_backward(
-    res: ForwardResult, grads: Sequence[Tensor | None], dests: Sequence[Tensor | None]
-) -> None:
-    """Per-position gradient of the pooled features of a forward (one launch).
-
-    ``grads[f]`` is the upstream gradient of feature f's pooled output and
-    ``dests[f]`` a contiguous ``[num_ids_f, dim]`` tensor of the weight dtype
-    that receives ``grad[bag] * w_i / max(count, 1)`` (mean) or
-    ``grad[bag] * w_i`` (sum) for every id position i; None skips feature f.
-    The forward must have kept its bag counts.
-    """
-
-    if res.bag_count is None or res.offsets is None:
-        raise RuntimeError("the forward ran without bag counts")
-    feats = res.feats.copy()
-    keep: list[Tensor] = []
-    sel: list[int] = []
-    for f, spec in enumerate(res.plan.features):
-        d = dests[f]
-        if d is None or spec.pooling == MDL_POOL_NONE:
-            continue
-        weight = res.plan.tables[spec.table].weight
-        n_f = int(feats["num_ids"][f])
-        dim = int(feats["dim"][f])
-        if d.dtype != weight.dtype or not d.is_contiguous() or d.numel() != n_f * dim:
-            raise ValueError("pool_backward destinations are contiguous [num_ids, dim] tensors of the weight dtype")
-        g = grads[f]
-        if g is None:
-            g = torch.zeros_like(res.outputs[f])
-        if g.dtype != spec.out_dtype:
-            g = g.to(spec.out_dtype)
-        if g.ndim != 2 or g.stride(-1) != 1:
-            g = g.reshape(-1, dim).contiguous()
-        keep.append(g)
-        feats["out"][f] = g.data_ptr()
-        feats["out_stride"][f] = g.stride(0)
-        feats["weight"][f] = d.data_ptr()
-        sel.append(f)
-    if not sel:
-        return
-    sub = np.ascontiguousarray(feats[sel])
-    target = forward_target_ids(sub)
-    n_chunks = lib().mdl_plan_chunks(sub.ctypes.data, len(sub), target, None, 0)
-    if n_chunks < 0:
-        check(int(n_chunks), "mdl_plan_chunks")
-    chunks = np.zeros(max(n_chunks, 1), dtype=CHUNK_DTYPE)
-    lib().mdl_plan_chunks(sub.ctypes.data, len(sub), target, chunks.ctypes.data, n_chunks)
-    device = res.device
-    sub_dev = upload(sub, device)
-    chunks_dev = upload(chunks, device)
-    ids_arg = res.ids if res.ids.numel() else res.keep[-1]
-    check(
-        lib().mdl_pool_backward(
-            sub_dev.data_ptr(), len(sub), chunks_dev.data_ptr(), n_chunks, ids_arg.data_ptr(), res.ids.numel(),
-            res.offsets.data_ptr(), res.bag_count.data_ptr(), feature_classes(sub), _stream(device),
-        ),
-        "mdl_pool_backward",
-    )
-    del keep
 
 
 def _segments(res: ForwardResult, feats: np.ndarray) -> list[tuple[KeyGroup, np.ndarray, int, int]]:
