@@ -352,7 +352,8 @@ int mdl_clamp_lengths(const uint64_t* lengths, const int64_t* rows, const int64_
  * payload) and (keys_alt, payload_alt).  *result_in_alt (host) is set to 1
  * when the sorted pairs end in the _alt buffers.  Equal keys keep input
  * order, so the segment reduction that follows sums duplicates in a fixed
- * order (deterministic), unlike the fp32-atomic index_add_ of the reference (src/optim.py:321-324 coalesce).
+ * order (deterministic), unlike the fp32-atomic index_add_ of the reference
+ * (src/optim.py:321-324 coalesce).
  */
 size_t mdl_sort_workspace_bytes(int64_t n);
 int mdl_sort_pairs(uint32_t* keys, uint32_t* payload, uint32_t* keys_alt,

@@ -9,18 +9,19 @@
 // class x lane width) are contiguous and each table's chunks consecutive.
 //
 // One wavefront reduces one chunk.  Its G = 64/L lane groups ("slots", L
-// lanes per row) each walk a contiguous slice of up to kSlotRun (48) entries
+// lanes per row) each walk a contiguous slice of about kSlotRun (48) entries
 // (fewer in a small call, see slot_run_for), accumulating the per-id gradients
-// in registers: the gradient rows of the slice are the only per-entry work, and a run that ends inside the slot that
-// began it is finished right there -- its summed gradient goes straight into
-// the Adagrad update, with the weight row and accumulator loaded alongside
-// the gradient rows (read and written once).  Runs that cross slot bounds are
-// joined once per chunk by a segmented scan over the slots' open partials.
-// A run that crosses chunk bounds (hot Zipf rows can have 10^4+ entries)
-// leaves one fp32 partial per chunk it touches; a second kernel adds those in
-// an order fixed by the chunk count and finishes the run.  The summation order depends on the
-// chunk layout only, and no floating-point atomics are used, so results do
-// not depend on scheduling.
+// in registers: the gradient rows of the slice are the only per-entry work,
+// and a run that ends inside the slot that began it is finished right there
+// -- its summed gradient goes straight into the Adagrad update, with the
+// weight row and accumulator loaded alongside the gradient rows (read and
+// written once).  Runs that cross slot bounds are joined once per chunk by a
+// segmented scan over the slots' open partials.  A run that crosses chunk
+// bounds (hot Zipf rows can have 10^4+ entries) leaves one fp32 partial per
+// chunk it touches; a second kernel adds those in an order fixed by the chunk
+// count and finishes the run.  The summation order depends on the chunk
+// layout only, and no floating-point atomics are used, so results do not
+// depend on scheduling.
 #include <mutex>
 
 #include "common.cuh"
@@ -83,18 +84,21 @@ struct BwdWs {
   float* chunk_ss;        // [max_chunks] squared norms of the runs finished per chunk
 };
 
-// Entries one slot walks in a full chunk: kSlotRun for a big call; a smaller
-// one takes shorter slices (one entry per kSlotTarget, down to kSlotRunMin),
+// Entries per slot of a full chunk: kSlotRun for a big call; a smaller one
+// takes fewer (one per kSlotTarget entries of the call, down to kSlotRunMin),
 // since a wave's walk is a chain of memory round trips and a small call has
-// waves to spare.  Reduce launches at one entry per 16 K / 32 K / 64 K / 128 K:
+// waves to spare.  A slice's length is the next odd number (see
+// reduce_chunk_body): 4 entries per slot are walked five at a time by four
+// fifths of the slots, 2 three at a time by two thirds, 48 by 47 of 48.
+// Reduce launches at one entry per 16 K / 32 K / 64 K / 128 K:
 // 393 K entries of 32 fp32 tables x 64 58.3 / 57.2 / 51.1 / 53.8 us (54.1
 // with slices of 16 at least); 893 K of 64 bf16 tables 80.9 / 55.3 / 40.5 /
 // 40.8 (its norm pass 49.3 / 29.5 / 21.6 / 23.9); 262 K of one bf16 table
 // 27.1 / 19.5 / 16.5 / 16.4 (27.4 with slices of 16 at least); 131 K uniform
 // ids 22.2 / 19.7 / 19.6 / 19.7 (29.2).  Shorter slices leave more runs
 // crossing slots and chunks; only the smallest calls, whose chunks leave most
-// CUs without a wave, gain from two entries (3 K entries 11.7 -> 9.3 us; 131 K
-// 19.5 -> 21.4).
+// CUs without a wave, gain from two entries per slot (3 K entries 11.7 -> 9.3
+// us; 131 K 19.5 -> 21.4).
 constexpr int kSlotRunMin = 4;
 constexpr int kSlotRunTiny = 2;
 constexpr int64_t kTinyEntries = 16384;
@@ -204,12 +208,7 @@ __global__ __launch_bounds__(kBoundThreads) void bwd_bounds_kernel(const mdl_tab
                                                                    const uint32_t* __restrict__ keys, int64_t n_cap,
                                                                    const int64_t* __restrict__ n_dev,
                                                                    int64_t* table_start, int64_t* table_end) {
-  // Sorted entries present: n_cap, or the caller's device count (clamped).
-  int64_t n = n_cap;
-  if (n_dev != nullptr) {
-    const int64_t c = *n_dev;
-    n = c < 0 ? 0 : (c > n_cap ? n_cap : c);
-  }
+  const int64_t n = entries_present(n_cap, n_dev);
   const int32_t t = blockIdx.x >> 1;
   const bool upper = blockIdx.x & 1;
   const uint64_t key = (uint64_t)tables[t].row_base + (upper ? (uint64_t)tables[t].num_rows : 0ull);
@@ -1308,7 +1307,9 @@ static int prepare(const mdl_table* tables, int32_t T, int32_t max_dim, uint32_t
       a.keys_out = const_cast<uint32_t*>(*sk);
       a.vals_out = const_cast<uint32_t*>(*sv);
       a.tile_min = nullptr;
-      // (a shorter tile ranks fewer slots)
+      // (a shorter tile ranks fewer slots: 1024 entries 14.5 us in a full
+      // tile's kernel, 9.1 in a quarter's; 2048 14.8, 11.6 in a half's; 3072
+      // 15.2, 13.4 in three quarters'; 4096 15.4)
       auto* kernel = n <= kMergeTile / 4       ? tile_plan_kernel<kTileItems / 4>
                      : n <= kMergeTile / 2     ? tile_plan_kernel<kTileItems / 2>
                      : n <= kMergeTile / 4 * 3 ? tile_plan_kernel<kTileItems / 4 * 3>

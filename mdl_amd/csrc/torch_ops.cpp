@@ -1650,11 +1650,11 @@ std::tuple<Tensor, Tensor> bucketize_cuda(const Tensor& raw_in, const std::optio
 // in one int64 buffer, the count (int32) after the last offset, when `joined`
 // -- a caller that reads both copies their two words at once.
 std::tuple<Tensor, Tensor, Tensor, Tensor> truncate_bags(const Tensor& values_in, const Tensor& offsets_in,
-                                                             const std::optional<Tensor>& valid_in,
-                                                             const std::optional<Tensor>& row_valid_in,
-                                                             int64_t max_length, c10::string_view truncation,
-                                                             c10::string_view bucket, int64_t num_buckets,
-                                                             bool validate_nonzero, bool joined) {
+                                                         const std::optional<Tensor>& valid_in,
+                                                         const std::optional<Tensor>& row_valid_in,
+                                                         int64_t max_length, c10::string_view truncation,
+                                                         c10::string_view bucket, int64_t num_buckets,
+                                                         bool validate_nonzero, bool joined) {
   require_device(values_in, "list values");
   TORCH_CHECK_TYPE(values_in.scalar_type() == at::kLong && offsets_in.scalar_type() == at::kLong,
                    "list values and offsets must be torch.int64");
@@ -2032,11 +2032,11 @@ void backward_sort_(const Tensor& tables, int64_t num_tables, const Tensor& keys
                     int64_t key_bits, const Tensor& ws, int64_t hints) {
   const at::Device dev = keys.device();
   const c10::DeviceGuard guard(dev);
-  check(mdl_backward_sort_hinted(reinterpret_cast<const mdl_table*>(tables.data_ptr()), (int32_t)num_tables, (int32_t)max_dim,
-                          reinterpret_cast<uint32_t*>(keys.data_ptr()), reinterpret_cast<uint32_t*>(payload.data_ptr()),
-                          num_entries,
-                          count.has_value() && count->defined() ? at_offset<int64_t>(*count, count_offset) : nullptr,
-                          (int32_t)key_bits, (uint32_t)hints, ws.data_ptr(), (size_t)ws.numel(), stream_of(dev)),
+  check(mdl_backward_sort_hinted(
+            reinterpret_cast<const mdl_table*>(tables.data_ptr()), (int32_t)num_tables, (int32_t)max_dim,
+            reinterpret_cast<uint32_t*>(keys.data_ptr()), reinterpret_cast<uint32_t*>(payload.data_ptr()), num_entries,
+            count.has_value() && count->defined() ? at_offset<int64_t>(*count, count_offset) : nullptr,
+            (int32_t)key_bits, (uint32_t)hints, ws.data_ptr(), (size_t)ws.numel(), stream_of(dev)),
         "mdl_backward_sort");
 }
 
