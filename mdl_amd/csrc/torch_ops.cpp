@@ -2211,3 +2211,12 @@ TORCH_LIBRARY_IMPL(mdl_hip, CPU, m) {
   m.impl("pool_bags_forward", &pool_bags_forward);
   m.impl("pool_bags_backward", &pool_bags_backward);
 }
+
+// These are called below autograd (inside an autograd function, or on whole
+// numbers); the dispatcher's boxed fallback for a missing autograd kernel cost
+// the pooling 2 us a call.
+TORCH_LIBRARY_IMPL(mdl_hip, Autograd, m) {
+  m.impl("bag_truncate_exact", torch::CppFunction::makeFallthrough());
+  m.impl("pool_bags_forward", torch::CppFunction::makeFallthrough());
+  m.impl("pool_bags_backward", torch::CppFunction::makeFallthrough());
+}
